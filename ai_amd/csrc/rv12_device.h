@@ -49,6 +49,18 @@ __device__ __forceinline__ void unpack_pairs(uint32_t d0, uint32_t d1, uint32_t 
            ((d2 << 1) & 0x80008000u);
 }
 
+// the same weights as float16 pairs: c is the exponent field (bias 15) and the
+// mantissa is padded with zeros, so the float16 value is the weight times
+// 2^(112 - sc), exactly (c = 0, the subnormals of base 0, included: both
+// formats read exponent field 0 at the scale of 1)
+__device__ __forceinline__ void unpack_pairs_f16(uint32_t d0, uint32_t d1, uint32_t d2, uint32_t p[4]) {
+    p[0] = (d0 & 0x80008000u) | ((d0 << 3) & 0x3FF83FF8u);
+    p[1] = (d1 & 0x80008000u) | ((d1 << 3) & 0x3FF83FF8u);
+    p[2] = (d2 & 0x80008000u) | ((d2 << 3) & 0x3FF83FF8u);
+    p[3] = ((d0 >> 8) & 0x00780078u) | ((d1 >> 4) & 0x07800780u) | (d2 & 0x38003800u) | ((d2 << 1) & 0x80008000u);
+}
+constexpr int kF16WeightExp = 112;  // float16 view over bf16 view of an h value: 2^112
+
 __device__ __forceinline__ float lo_f(uint32_t p) { return __uint_as_float(p << 16); }
 __device__ __forceinline__ float hi_f(uint32_t p) { return __uint_as_float(p & 0xFFFF0000u); }
 
@@ -130,6 +142,28 @@ __device__ __forceinline__ void split3(const float (&v)[8], u32x4& hi, u32x4& mi
     hi = u32x4{h[0] | h[1] << 16, h[2] | h[3] << 16, h[4] | h[5] << 16, h[6] | h[7] << 16};
     mid = u32x4{m[0] | m[1] << 16, m[2] | m[3] << 16, m[4] | m[5] << 16, m[6] | m[7] << 16};
     lo = u32x4{l[0] | l[1] << 16, l[2] | l[3] << 16, l[4] | l[5] << 16, l[6] | l[7] << 16};
+}
+
+// split 8 values into two float16x8 parts, hi + lo = v to 22 bits (a residual
+// below 2^-14 loses what is below 2^-24)
+__device__ __forceinline__ void split2_f16(const float (&v)[8], u32x4& hi, u32x4& lo) {
+    uint32_t h[8], l[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        const _Float16 a = (_Float16)v[e];
+        h[e] = (uint32_t)__builtin_bit_cast(uint16_t, a);
+        l[e] = (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)(v[e] - (float)a));
+    }
+    hi = u32x4{h[0] | h[1] << 16, h[2] | h[3] << 16, h[4] | h[5] << 16, h[6] | h[7] << 16};
+    lo = u32x4{l[0] | l[1] << 16, l[2] | l[3] << 16, l[4] | l[5] << 16, l[6] | l[7] << 16};
+}
+
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+
+// one v_mfma_f32_16x16x32_f16 (the lane layout of the bf16 one)
+__device__ __forceinline__ f32x4 mfma_f16(u32x4 a, u32x4 b, f32x4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0,
+                                                  0);
 }
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));

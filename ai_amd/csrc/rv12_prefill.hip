@@ -1,39 +1,41 @@
-// rv12 prefill linear: the 12-bit decode fused into a bf16x3 MFMA GEMM over
-// all the prompt's tokens at once (gfx950).  Replaces the blocked prefill's
-// decode_rows + fp32 GEMM (ramvi/engine/ramvi_engine/kernels/prefill.py:66-78,
-// prefill_kernels.py:8-26 and 58-110): every weight is read once per prompt
-// in its 12-bit form, never written back in a wider format.
+// rv12 prefill linear: the 12-bit decode fused into a split-float16 MFMA GEMM
+// over all the prompt's tokens at once (gfx950).  Replaces the blocked
+// prefill's decode_rows + fp32 GEMM
+// (ramvi/engine/ramvi_engine/kernels/prefill.py:66-78, prefill_kernels.py:8-26
+// and 58-110): every weight is read once per prompt in its 12-bit form, never
+// written back in a wider format.
 //
 // y[t] (=|+=) W_dec . x'[t], t < T, with the MODE prologue (2: x' =
 // silu(x[0:K]) * x[K:2K]) or the RMSNorm prologue of mode 0 (x' = lnw x,
 // the token's rs = 1 / sqrt(mean x^2 + eps) applied to its outputs, as the
-// decode kernels apply it).  Three launches:
-//   1. k_prefill_stats (one wave per token): each token's exponent scale
-//      P_t (64 when its largest |x'| lies in [2^-40, 2^63), else 100 minus
-//      the exponent of the largest) and, with RMS, its rs (sum of squares of
-//      x 2^-32); k_prefill_parts (32 tokens x 64 columns per workgroup):
-//      x' 2^P_t split into bf16 parts
-//      hi + mid + lo (24 significand bits, as the reference's _x3 split,
-//      wcomp.py:130-140) in B-operand lane order: for token block tb, step
-//      s (32 columns) and part, 64 lanes x 8 bf16 (lane l: token l%16,
-//      k = 8(l/16) + 0..7), and x' itself in fp32, transposed (column-major
-//      over the padded tokens).  Token rows past T are zeros.
-//   2. k_prefill_mm: workgroup = 256 rows x 128 tokens, 8 waves of 64 rows x
-//      64 tokens.  Per 32-column step the workgroup's 16 row blocks' Q16
-//      tiles (the A operand of v_mfma_f32_16x16x32_bf16, the h values
-//      w 2^-sc) and the B parts of its 8 token blocks go from memory straight
-//      into a ring of four LDS slots (buffer loads with the LDS destination;
-//      no register holds them on the way, every wait is explicit), three
-//      steps ahead; one wait + barrier per step; each wave reads the next
-//      step's fragments while its 48 MFMAs of the current step run; the MFMAs
-//      accumulate in 16 independent fp32 accumulators.  Epilogue:
-//      v = acc 2^(sc_row - P_t) (exact); the packed form's exception entries
-//      of the wave's rows (weights outside a row's window, zeros in the
-//      tiles) add ev * x'[t][col] in list order, x' read from the transposed
-//      copy (one column of the wave's 64 tokens is 256 contiguous bytes,
-//      where the rows of x would take a cache line per token); with RMS v is
-//      scaled by rs_t; then y is stored or added; rows past N and tokens past
-//      T are skipped.
+// decode kernels apply it).  Three launches, four with a K split:
+//   1. k_prefill_stats (one wave per token): the exponents of x' and, with
+//      RMS, rs (sum of squares of x 2^-32); k_prefill_parts (32 tokens x 64
+//      columns per workgroup): x' 2^P_t split into parts in B-operand lane
+//      order (token block, step of 32 columns, part, 64 lanes x 8 values; lane
+//      l: token l%16, k = 8(l/16) + 0..7), and x' itself in fp32, transposed
+//      (column-major over the padded tokens).  Token rows past T are zeros.
+//   2. k_prefill_mm: a 12-bit weight is exactly a float16 (4 exponent bits, 7
+//      of mantissa), so x' needs two float16 parts (22 bits) and two MFMAs per
+//      tile where three bf16 parts (24 bits) took three; the sums pass from
+//      the matrix core's accumulators to fp32 ones every kPfChunk steps and come
+//      out closer to 64 bits than before (24576 x 4096 over 2048 tokens:
+//      relative error 7.0e-7 -> 2.3e-7; 1024 x 3072 over 301: 1.95e-7 ->
+//      1.79e-7).  A tile with a token whose values the float16 parts would not
+//      hold (see tok_exp) keeps the three bf16 parts.
+//      Workgroup = 256 rows x 128 tokens, 8 waves of 64 rows x 64 tokens.  Per
+//      32-column step the workgroup's 16 row blocks' Q16 tiles and the B parts
+//      go from memory straight into a ring of LDS slots (buffer loads with the
+//      LDS destination), one wait + barrier per step; every other instruction
+//      is spread between the MFMAs.
+//      Bound by the matrix cores at the clock that the power limit leaves:
+//      51200 x 5120 over 4096 tokens is 2.15e12 useful operations and twice
+//      that in MFMAs, 5560 us with three parts and 4000 with two: the matrix
+//      cores are busy about half of the cycles at 1.8 GHz, and a library's
+//      bf16 product of that shape reaches 1.17 PFLOP/s where this does 1.07.
+//      (256-token workgroups, whose waves read a sixth less from LDS per
+//      product, took 3590 us, but leave no registers for the second sums:
+//      their error stays at 5.9e-7.)
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -43,32 +45,63 @@
 namespace rv12 {
 
 constexpr int kPfRowBlocks = 16;  // row blocks (of 16 rows) per workgroup
-constexpr int kPfTokBlocks = 8;   // token blocks (of 16 tokens) per workgroup
 constexpr int kPfThreads = 512;
-// wave tile: kPfWB row blocks x kPfWT token blocks (8 waves: 16 / kPfWB along
-// the rows times 8 / kPfWT along the tokens)
-constexpr int kPfWB = 4;
-constexpr int kPfWR = kPfRowBlocks / kPfWB;                          // waves along the rows
-constexpr int kPfWT = kPfTokBlocks / (kPfThreads / 64 / kPfWR);  // token blocks per wave
-static_assert(kPfWR * (kPfTokBlocks / kPfWT) == kPfThreads / 64, "8 waves cover the workgroup tile");
-constexpr int kPfRing = 4;  // LDS slots: the A tiles and B parts of steps s .. s + 3
-// slot layout (u32x4 units): 16 A tiles of 1 KB (a 12-byte-per-lane load with
-// the LDS destination writes lane l at 16 l: 768 B of each KB), then the B
-// parts (8 token blocks x 3 parts x 64 lanes)
+constexpr int kPfWaves = kPfThreads / 64;
+// wave tile: kPfWB row blocks x kPfWT token blocks; kPfWR waves along the rows,
+// kPfWC along the tokens
+constexpr int kPfWB = 4, kPfWT = 4;
+constexpr int kPfWR = kPfRowBlocks / kPfWB;
+constexpr int kPfWC = kPfWaves / kPfWR;
+constexpr int kPfTokBlocks = kPfWC * kPfWT;           // token blocks (of 16 tokens) per workgroup
+constexpr int kPfTokens = kPfTokBlocks * 16;          // 128
+constexpr int kPfAPerWave = kPfRowBlocks / kPfWaves;  // A tiles a wave loads per step
+// LDS slot (u32x4 units): 16 A tiles of 1 KB (a 12-byte-per-lane load with the
+// LDS destination writes lane l at 16 l: 768 B of each KB), then the B parts
+// (64 lanes each per token block)
 constexpr int kPfSlotA = kPfRowBlocks * 64;
-constexpr int kPfSlot = kPfSlotA + kPfTokBlocks * 3 * 64;  // 40 KB
-constexpr size_t kPfLds = (size_t)kPfRing * kPfSlot * 16;   // 160 KB
-static_assert(kPfLds <= 160 * 1024, "gfx950 LDS per workgroup");
-// loads a wave issues per step: 2 A tiles and 3 B chunks, all into LDS
-constexpr int kPfOpsPerStep = kPfRowBlocks / (kPfThreads / 64) + 3;
-// at the top of step s, the wave's loads of step s + 1 (issued at step
-// s + 1 - kPfRing) are followed by those of the kPfRing - 2 steps between
-constexpr int kPfWait = kPfOpsPerStep * (kPfRing - 2);
-static_assert(kPfWait < 64, "vmcnt holds 6 bits");
+constexpr size_t kPfLds = 160 * 1024;  // the whole CU's: one workgroup per CU
+// a wave's sums of 64 rows x 64 tokens on their way past the exceptions, rows
+// 68 floats apart (the four row groups of an access fall on different banks)
+constexpr int kPfExcStride = 68;
+static_assert((size_t)kPfWaves * 16 * kPfWB * kPfExcStride * 4 <= kPfLds, "LDS");
+// float16 loop: 2 parts, a ring of five 32 KB slots
+constexpr int kPfSlot2 = kPfSlotA + kPfTokBlocks * 2 * 64;
+constexpr int kPfRing2 = (int)(kPfLds / (kPfSlot2 * 16));
+static_assert(kPfRing2 == 5, "five slots");
+constexpr int kPfB2 = kPfTokBlocks * 2 / kPfWaves;  // 1 KB chunks of B a wave loads per step
+constexpr int kPfOps2 = kPfAPerWave + kPfB2;
+// at the top of step s, the wave's loads of step s + 1 are followed by those
+// of the kPfRing2 - 3 steps issued since
+constexpr int kPfWait2 = kPfOps2 * (kPfRing2 - 3);
+// Steps between the additions of the MFMA accumulators to the fp32 sums.  The
+// matrix core's own additions into an accumulator lose more as it grows: all
+// 128 steps of K = 4096 in one accumulator leave a relative error of 5.9e-7
+// against 64 bits (7.0e-7 with three bf16 parts), chunks of 16 steps 2.3e-7,
+// of 8 1.9e-7, of 4 1.7e-7; 51200 x 5120 over 4096 tokens takes 4310, 4115,
+// 4170 and 4290 us.
+constexpr int kPfChunk = 16;
+// bf16 loop: 3 parts, four 40 KB slots
+constexpr int kPfRing3 = 4;
+constexpr int kPfSlot3 = kPfSlotA + kPfTokBlocks * 3 * 64;
+static_assert((size_t)kPfRing3 * kPfSlot3 * 16 <= kPfLds, "LDS of one workgroup");
+constexpr int kPfOps3 = kPfAPerWave + kPfTokBlocks * 3 / kPfWaves;
+constexpr int kPfWait3 = kPfOps3 * (kPfRing3 - 1);  // the loads issued after step s's
+static_assert(kPfWait3 < 64 && kPfWait2 < 64, "vmcnt holds 6 bits");
 // s_waitcnt immediates (gfx9 encoding): vmcnt(n) and lgkmcnt(0), expcnt not
 // waited for; vmcnt(n) alone
 constexpr int waitcnt_vm_lgkm0(int n) { return (n & 15) | ((n >> 4) << 14) | (7 << 4); }
 constexpr int waitcnt_vm(int n) { return waitcnt_vm_lgkm0(n) | (15 << 8); }
+constexpr int waitcnt_lgkm0() { return waitcnt_vm_lgkm0(63); }
+
+// 12 or 16 bytes per lane from a descriptor straight into LDS (lane l at
+// d + 16 bytes l)
+typedef __attribute__((address_space(3))) void* lds_ptr;
+__device__ __forceinline__ void load_lds12(__amdgpu_buffer_rsrc_t r, u32x4* d, int off, int soff) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_ptr)d, 12, off, soff, 0, 0);
+}
+__device__ __forceinline__ void load_lds16(__amdgpu_buffer_rsrc_t r, u32x4* d, int off, int soff) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_ptr)d, 16, off, soff, 0, 0);
+}
 
 // x' of token row xr at columns k..k+7 (MODE 2: silu(g) * u; lnw: the RMS
 // weight times x)
@@ -95,17 +128,43 @@ __device__ __forceinline__ void prefill_xprime(const float* xr, int K, int k, bo
     }
 }
 
+// A token's activation class, E = e << 1 | wide: e the largest exponent of
+// its finite nonzero |x'| (-1000: none), wide where the float16 split would
+// hold fewer bits of it than the float32 sums keep.  The float16 parts are of
+// x' 2^(15 - e): 22 bits of each value, and nothing below 2^-39 of the largest.
+// Where the mean exponent of the token's nonzero values is at least e - 14, the
+// root mean square of x' is at least 2^-15 of the largest (the geometric mean
+// is below it), so the second part is below 2^-24 of it; other tokens (a few
+// huge values among tiny ones) are wide and keep the three bf16 parts, as
+// does every token of their tile.
+constexpr int kF16MeanBelow = 14;
+__device__ __forceinline__ int tok_exp(int E) { return E >> 1; }
+__device__ __forceinline__ int scale_f16(int E) { return tok_exp(E) < -500 ? 0 : 15 - tok_exp(E); }
+__device__ __forceinline__ int scale_bf16(int E) {
+    const int e = tok_exp(E);
+    return (e >= -39 && e <= kXRangeHi) ? kXScaleExp : slow_scale_exp(e);
+}
+
+// any of the tile's tokens t0 .. t0 + 127 below T is wide (t0 < T): the lanes'
+// part of the answer, a ballot of bit 0 away from the whole
+__device__ __forceinline__ int wide_lanes(const int* __restrict__ E, int t0, int T) {
+    int any = 0;
+#pragma unroll
+    for (int i = 0; i < kPfTokens; i += 64) any |= E[min(t0 + i + (int)(threadIdx.x & 63), T - 1)];
+    return any;
+}
+
 // 1a. k_prefill_stats: one wave per token (4 per workgroup, a grid over the
-// padded tokens): the largest exponent of |x'| and, with RMS, the sum of
-// squares of x 2^-32, lane l over columns 8 l + 512 i, reduced across the
-// wave in a fixed order; writes the token's scale exponent P_t and rs_t.
+// padded tokens): the largest exponent of |x'|, the sum of its exponents and,
+// with RMS, the sum of squares of x 2^-32, lane l over columns 8 l + 512 i,
+// reduced across the wave in a fixed order; writes the token's E and rs_t.
 constexpr int kPsThreads = 256;
 __global__ __launch_bounds__(kPsThreads) void k_prefill_stats(const float* __restrict__ x, int T, int K, int xs,
                                                               int m2, const uint16_t* __restrict__ lnw, float eps,
-                                                              int* __restrict__ P, float* __restrict__ R) {
+                                                              int* __restrict__ E, float* __restrict__ R) {
     const int lane = threadIdx.x & 63;
     const int t = blockIdx.x * (kPsThreads / 64) + (threadIdx.x >> 6);
-    int e = -1000;
+    int e = -1000, cnt = 0, es = 0;  // |es| <= 2^20 columns x 149
     float sq = 0.0f;
     if (t < T) {
         const float* xr = x + (int64_t)t * xs;
@@ -124,16 +183,25 @@ __global__ __launch_bounds__(kPsThreads) void k_prefill_stats(const float* __res
                 }
             }
 #pragma unroll
-            for (int i = 0; i < 8; ++i) e = max(e, exp_or_min(v[i]));
+            for (int i = 0; i < 8; ++i) {
+                const int ei = exp_or_min(v[i]);
+                const bool ok = ei > -1000;
+                e = max(e, ei);
+                cnt += ok ? 1 : 0;
+                es += ok ? ei : 0;
+            }
         }
     }
 #pragma unroll
     for (int o = 32; o >= 1; o >>= 1) {
         e = max(e, __shfl_xor(e, o));
+        cnt += __shfl_xor(cnt, o);
+        es += __shfl_xor(es, o);
         sq += __shfl_xor(sq, o);
     }
     if (lane == 0) {
-        P[t] = (e >= -39 && e <= kXRangeHi) ? kXScaleExp : slow_scale_exp(e);
+        const bool wide = (int64_t)es < (int64_t)cnt * (e - kF16MeanBelow);
+        E[t] = e * 2 + (wide ? 1 : 0);
         if (lnw) R[t] = rms_scale(sq, K, eps);
     }
 }
@@ -141,35 +209,42 @@ __global__ __launch_bounds__(kPsThreads) void k_prefill_stats(const float* __res
 // 1b. k_prefill_parts: grid (32-token blocks, 64-column chunks), 256 threads,
 // thread (token tok, 8-column group k8): x' (prologue applied) of token t at
 // columns kc .. kc + 7 written transposed (per column, 32 consecutive tokens:
-// full 128-byte lines), then x' 2^P_t split into the bf16 parts in B-operand
-// lane order.  Tokens past T are zeros.
+// full 128-byte lines), then its scaled parts in B-operand lane order: two of
+// float16, or three of bf16 where a token of the GEMM's 128-token tile is wide.  Tokens past T are zeros.
 constexpr int kPpThreads = 256;
 __global__ __launch_bounds__(kPpThreads) void k_prefill_parts(const float* __restrict__ x, int T, int K, int xs,
                                                               int m2, const uint16_t* __restrict__ lnw,
-                                                              const int* __restrict__ P, u32x4* __restrict__ xb,
+                                                              const int* __restrict__ E, u32x4* __restrict__ xb,
                                                               float* __restrict__ xt, int tp) {
     const int tok = threadIdx.x & 31, k8 = threadIdx.x >> 5;
     const int t = blockIdx.x * 32 + tok;
     const int kc = blockIdx.y * 64 + k8 * 8;
-    if (kc >= K) return;
     const int nsteps = K >> 5;
     float v[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
-    if (t < T) prefill_xprime(x + (int64_t)t * xs, K, kc, m2 != 0, lnw, v);
+    if (t < T && kc < K) prefill_xprime(x + (int64_t)t * xs, K, kc, m2 != 0, lnw, v);
+    const bool wide = __ballot(wide_lanes(E, (int)(blockIdx.x * 32) / kPfTokens * kPfTokens, T) & 1) != 0;
+    if (kc >= K) return;
     float* xc = xt + (int64_t)kc * tp + t;
 #pragma unroll
     for (int i = 0; i < 8; ++i) xc[(int64_t)i * tp] = v[i];
-    u32x4 hi = {0, 0, 0, 0}, mid = {0, 0, 0, 0}, lo = {0, 0, 0, 0};
-    if (t < T) {
-        const int p = P[t];
+    const int p = t < T ? (wide ? scale_bf16(E[t]) : scale_f16(E[t])) : 0;
 #pragma unroll
-        for (int i = 0; i < 8; ++i) v[i] = ldexpf(v[i], p);
+    for (int i = 0; i < 8; ++i) v[i] = ldexpf(v[i], p);
+    const int s = kc >> 5, l = ((kc & 31) >> 3) * 16 + (t & 15);  // step, lane of the operand
+    u32x4* blk = xb + (int64_t)(t >> 4) * nsteps * 192;
+    u32x4 hi, mid, lo;
+    if (wide) {
         split3(v, hi, mid, lo);
+        u32x4* d = blk + (int64_t)s * 192 + l;
+        d[0] = hi;
+        d[64] = mid;
+        d[128] = lo;
+    } else {
+        split2_f16(v, hi, lo);
+        u32x4* d = blk + (int64_t)s * 128 + l;
+        d[0] = hi;
+        d[64] = lo;
     }
-    const int s = kc >> 5, g = (kc & 31) >> 3;  // step, 8-column group in the step
-    u32x4* d = xb + ((int64_t)(t >> 4) * nsteps + s) * 192 + g * 16 + (t & 15);
-    d[0] = hi;
-    d[64] = mid;
-    d[128] = lo;
 }
 
 // Workgroup i -> (row tile, token tile).  Workgroups are dispatched in order,
@@ -178,9 +253,9 @@ __global__ __launch_bounds__(kPpThreads) void k_prefill_parts(const float* __res
 // G / 8 tiles (the remainder past 8 (G / 8) keeps v = i), and v runs over
 // groups of kPfGroupRows row tiles x all token tiles, row tile fastest, so the
 // ~32 workgroups an XCD holds at once cover 8 row tiles x 4 token tiles: per
-// step their L2 misses are 8 A tiles (12 KB each) and 4 B sets (24 KB each),
-// 192 KB, where 2 row tiles x 16 token tiles (the Qwen3-8B o and down in
-// launch order) would miss 408 KB.  A bijection of [0, G).
+// step their L2 misses are 8 A tiles (12 KB each) and 4 B sets (16 KB each at
+// 128 tokens), 160 KB, where 2 row tiles x 16 token tiles (the Qwen3-8B o and
+// down in launch order) would miss 280 KB.  A bijection of [0, G).
 constexpr int kPfGroupRows = 8;
 __device__ __forceinline__ void prefill_tile(int i, int G, int nx, int ny, int& rt, int& tt) {
     const int g8 = G / 8;
@@ -200,14 +275,14 @@ __device__ __forceinline__ void prefill_tile(int i, int G, int nx, int ny, int& 
 template <bool LN>
 __global__ __launch_bounds__(kPfThreads) void k_prefill_mm(const uint32_t* __restrict__ tiles,
                                                            const int32_t* __restrict__ rbase,
-                                                           const u32x4* __restrict__ xb, const int* __restrict__ P,
+                                                           const u32x4* __restrict__ xb, const int* __restrict__ E,
                                                            const int32_t* __restrict__ rp,
                                                            const int32_t* __restrict__ er,
                                                            const int32_t* __restrict__ ec,
                                                            const float* __restrict__ ev, const float* __restrict__ xt,
                                                            int tp, const float* __restrict__ R, float* __restrict__ y,
                                                            float* __restrict__ part, int N, int K, int T, int add) {
-    extern __shared__ u32x4 bs[];  // [kPfRing][kPfSlot]: A tiles and B parts of steps s .. s + 3
+    extern __shared__ u32x4 bs[];  // the ring's slots: A tiles and B parts of consecutive steps
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wr = wave % kPfWR, wc = wave / kPfWR;
@@ -220,9 +295,11 @@ __global__ __launch_bounds__(kPfThreads) void k_prefill_mm(const uint32_t* __res
     int rt, tt;
     prefill_tile(blockIdx.x, gridDim.x, nx, gridDim.x / nx, rt, tt);
     const int64_t blk0 = (int64_t)rt * kPfRowBlocks + wr * kPfWB;  // this wave's first row block
-    const int tb0 = tt * kPfTokBlocks;                          // the workgroup's first token block
+    const int tb0 = tt * kPfTokBlocks;                            // the workgroup's first token block
     const uint32_t blk_bytes = (uint32_t)nsteps * kStepBytes;
-    typedef __attribute__((address_space(3))) void* lds_ptr;
+    // a wide token in the tile: the parts are three of bf16 (asked for here,
+    // answered after the first loads are on their way)
+    const int wl = wide_lanes(E, tb0 * 16, T);
     // the workgroup's A tiles: wave w loads row blocks 2w and 2w + 1 of the
     // workgroup through a descriptor over its valid row blocks (a row block
     // past N, or a step past the end through the 0-byte descriptor, reads
@@ -232,105 +309,186 @@ __global__ __launch_bounds__(kPfThreads) void k_prefill_mm(const uint32_t* __res
     const char* wgbase = reinterpret_cast<const char*>(tiles) + wblk0 * (int64_t)blk_bytes;
     const __amdgpu_buffer_rsrc_t rv = make_rsrc(wgbase, (uint32_t)nvalid_wg * blk_bytes);
     const __amdgpu_buffer_rsrc_t rnull = make_rsrc(wgbase, 0u);
-    constexpr int kAPerWave = kPfRowBlocks / (kPfThreads / 64);
-    int aoff[kAPerWave];
+    int aoff[kPfAPerWave];
 #pragma unroll
-    for (int i = 0; i < kAPerWave; ++i) aoff[i] = (int)((wave * kAPerWave + i) * blk_bytes) + lane * 12;
-    // the B parts of the workgroup's token blocks: 3 chunks of 64 lanes x
-    // 16 B per wave, through a descriptor over the workgroup's parts
+    for (int i = 0; i < kPfAPerWave; ++i) aoff[i] = (int)((wave * kPfAPerWave + i) * blk_bytes) + lane * 12;
+    // the B parts of the workgroup's token blocks, through a descriptor over them
     const u32x4* xbw = xb + (int64_t)tb0 * nsteps * 192;
     const __amdgpu_buffer_rsrc_t rbx = make_rsrc(xbw, (uint32_t)kPfTokBlocks * nsteps * 192 * 16);
     const __amdgpu_buffer_rsrc_t rbnull = make_rsrc(xbw, 0u);
-    int boff[3];
-#pragma unroll
-    for (int j = 0; j < 3; ++j) {
-        const int idx = tid + j * kPfThreads;  // (token block, part, lane) of the step
-        boff[j] = ((idx / 192) * nsteps * 192 + idx % 192) * 16;
-    }
-    // step s's A tiles and B parts into LDS slot `slot`; a step past the end
-    // goes through the 0-byte descriptors, which write zeros, so the loop has
-    // no branch around a load
-    auto load_step = [&](int slot, int j) {  // step s_lo + j
-        const int s = s_lo + j;
-        const bool in = s < s_hi;
-        const __amdgpu_buffer_rsrc_t ra = in ? rv : rnull, rb = in ? rbx : rbnull;
-        const int sa = (in ? s : 0) * kStepBytes, sb = (in ? s : 0) * 192 * 16;
-        u32x4* d = bs + slot * kPfSlot;
-#pragma unroll
-        for (int i = 0; i < kAPerWave; ++i)
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (lds_ptr)(d + (wave * kAPerWave + i) * 64), 12, aoff[i], sa,
-                                                     0, 0);
-#pragma unroll
-        for (int j = 0; j < 3; ++j)
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, (lds_ptr)(d + kPfSlotA + wave * 64 + j * kPfThreads), 16,
-                                                     boff[j], sb, 0, 0);
-    };
-    // this wave's fragments of the step in slot `slot`: its 4 row blocks' A
-    // groups (12 bytes per lane) and 3 parts x 4 token blocks of B,
-    // part-major so the first part's MFMAs wait only for its own reads
-    auto read_frags = [&](u32x3 (&ra)[kPfWB], u32x4 (&rb)[3][kPfWT], int slot) {
-        const u32x4* d = bs + slot * kPfSlot;
-#pragma unroll
-        for (int b = 0; b < kPfWB; ++b) ra[b] = *reinterpret_cast<const u32x3*>(d + (wr * kPfWB + b) * 64 + lane);
-        const u32x4* src = d + kPfSlotA + (wc * kPfWT) * 192 + lane;
-#pragma unroll
-        for (int q = 0; q < 3; ++q)
-#pragma unroll
-            for (int c = 0; c < kPfWT; ++c) rb[q][c] = src[c * 192 + q * 64];
-    };
 
     f32x4 acc[kPfWB][kPfWT];
 #pragma unroll
     for (int b = 0; b < kPfWB; ++b)
 #pragma unroll
         for (int c = 0; c < kPfWT; ++c) acc[b][c] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    // prologue: steps 0-3 into slots 0-3, all landed; step 0's fragments read
-#pragma unroll
-    for (int i = 0; i < kPfRing; ++i) load_step(i, i);
-    asm volatile("" ::: "memory");
-    __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-    u32x3 fa[2][kPfWB];
-    u32x4 fb[2][3][kPfWT];
-    read_frags(fa[0], fb[0], 0);
 
-    // Step s, software-pipelined: wait for this wave's loads of step s + 1
-    // and for its fragment reads of step s; barrier (every wave's loads of
-    // step s + 1 have landed, and every wave is done reading slot s % 4);
-    // step s + 4 into that slot; the fragments of step s + 1 read while the
-    // A groups of step s are unpacked and its 48 MFMAs run.  The loop runs
-    // whole rounds of the unroll: steps past the split read zeros (A and B) and
-    // add nothing.
-    const int nround = (s_hi - s_lo + kPfRing - 1) / kPfRing * kPfRing;
-    for (int s0 = 0; s0 < nround; s0 += kPfRing) {
+    constexpr int kFrags = 2 * kPfWT;
+    constexpr int W = 4;  // B fragments in flight (8: the same within 1 %)
+    int boff[kPfB2];
 #pragma unroll
-        for (int u = 0; u < kPfRing; ++u) {
-            const int s = s0 + u;
-            // (the empty asm statements keep every LDS access on its side of
-            // the wait and the barrier: neither builtin orders memory)
+    for (int j = 0; j < kPfB2; ++j) {
+        const int idx = tid + j * kPfThreads;  // (token block, part, lane) of the step
+        boff[j] = ((idx / 128) * nsteps * 192 + idx % 128) * 16;
+    }
+    // load i of step s_lo + j into the slot at `slot`; a step past the end
+    // goes through the 0-byte descriptors, which write zeros, so the loop
+    // has no branch around a load
+    auto load_op = [&](int i, int slot, int j) {
+        const int s = s_lo + j;
+        const bool in = s < s_hi;
+        u32x4* d = bs + slot;
+        if (i < kPfAPerWave)
+            load_lds12(in ? rv : rnull, d + (wave * kPfAPerWave + i) * 64, aoff[i], (in ? s : 0) * kStepBytes);
+        else
+            load_lds16(in ? rbx : rbnull, d + kPfSlotA + wave * 64 + (i - kPfAPerWave) * kPfThreads,
+                       boff[i - kPfAPerWave], (in ? s : 0) * 128 * 16);
+    };
+    // steps 0 .. kPfRing2 - 2 into slots 0 .. (a wide tile starts over: what these
+    // loads bring is in bounds and unused)
+#pragma unroll
+    for (int j = 0; j < kPfRing2 - 1; ++j)
+#pragma unroll
+        for (int i = 0; i < kPfOps2; ++i) load_op(i, j * kPfSlot2, j);
+    const bool wide = __ballot(wl & 1) != 0;
+
+    if (!wide) {
+        const int ra0 = wr * kPfWB * 64 + lane, rb0 = kPfSlotA + wc * kPfWT * 128 + lane;
+        auto read_a = [&](int slot, int b) { return *reinterpret_cast<const u32x3*>(bs + slot + ra0 + b * 64); };
+        // fragment i: part i / kPfWT of token block i % kPfWT, so that the products
+        // of one accumulator are kPfWT fragments apart
+        auto read_b = [&](int slot, int i) { return bs[slot + rb0 + (i % kPfWT) * 128 + (i / kPfWT) * 64]; };
+        // steps 0 and 1 landed
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_waitcnt(waitcnt_vm(kPfWait2));
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        u32x4 a[2][kPfWB], fb[W];
+#pragma unroll
+        for (int b = 0; b < kPfWB; ++b) {
+            const u32x3 r = read_a(0, b);
+            uint32_t pr[4];
+            unpack_pairs_f16(r.x, r.y, r.z, pr);
+            a[0][b] = u32x4{pr[0], pr[1], pr[2], pr[3]};
+        }
+#pragma unroll
+        for (int i = 0; i < W; ++i) fb[i] = read_b(0, i);
+        // Step s: wait for this wave's loads of step s + 1; barrier (every
+        // wave's have landed, and every wave has used slot s - 1); then per B
+        // fragment its four MFMAs, one of the loads of step s + kPfRing2 - 1 into
+        // slot s - 1, the read of the fragment W ahead (the next step's at the
+        // end) and a share of the next step's A reads and unpacking: memory,
+        // LDS and vector instructions spread between the MFMAs, fenced so
+        // that the compiler keeps them there.
+        int cur = 0, nxt = kPfSlot2, fill = (kPfRing2 - 1) * kPfSlot2;
+        const int nst = s_hi - s_lo;
+        f32x4 sum[kPfWB][kPfWT];
+#pragma unroll
+        for (int b = 0; b < kPfWB; ++b)
+#pragma unroll
+            for (int c = 0; c < kPfWT; ++c) sum[b][c] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        for (int s1 = 0; s1 < nst; s1 += kPfChunk) {
+            const int s2 = min(nst, s1 + kPfChunk);
+            for (int s0 = s1; s0 < s2; s0 += 2) {
+#pragma unroll
+                for (int u = 0; u < 2; ++u) {
+                    asm volatile("" ::: "memory");
+                    __builtin_amdgcn_s_waitcnt(waitcnt_vm(kPfWait2));
+                    __builtin_amdgcn_s_barrier();
+                    asm volatile("" ::: "memory");
+                    u32x3 raw[kPfWB];
+#pragma unroll
+                    for (int i = 0; i < kFrags; ++i) {
+                        if (i < kPfOps2) load_op(i, fill, s0 + u + kPfRing2 - 1);
+                        if (i < kPfWB) raw[i] = read_a(nxt, i);
+                        const u32x4 bf = fb[i % W];
+#pragma unroll
+                        for (int b = 0; b < kPfWB; ++b) acc[b][i % kPfWT] = mfma_f16(a[u][b], bf, acc[b][i % kPfWT]);
+                        fb[i % W] = i + W < kFrags ? read_b(cur, i + W) : read_b(nxt, i + W - kFrags);
+                        if (i >= kFrags - kPfWB) {
+                            const int b = i - (kFrags - kPfWB);
+                            uint32_t pr[4];
+                            unpack_pairs_f16(raw[b].x, raw[b].y, raw[b].z, pr);
+                            a[u ^ 1][b] = u32x4{pr[0], pr[1], pr[2], pr[3]};
+                        }
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+                    fill = cur;
+                    cur = nxt;
+                    nxt = nxt + kPfSlot2 == kPfRing2 * kPfSlot2 ? 0 : nxt + kPfSlot2;
+                }
+            }
+#pragma unroll
+            for (int b = 0; b < kPfWB; ++b)
+#pragma unroll
+                for (int c = 0; c < kPfWT; ++c) {
+                    sum[b][c] += acc[b][c];
+                    acc[b][c] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+                }
+        }
+#pragma unroll
+        for (int b = 0; b < kPfWB; ++b)
+#pragma unroll
+            for (int c = 0; c < kPfWT; ++c) acc[b][c] = sum[b][c];
+    } else {
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        int boff3[3];
+#pragma unroll
+        for (int j = 0; j < 3; ++j) {
+            const int idx = tid + j * kPfThreads;  // (token block, part, lane) of the step
+            boff3[j] = ((idx / 192) * nsteps * 192 + idx % 192) * 16;
+        }
+        auto load_step = [&](int slot, int j) {  // step s_lo + j
+            const int s = s_lo + j;
+            const bool in = s < s_hi;
+            const __amdgpu_buffer_rsrc_t ra = in ? rv : rnull, rb = in ? rbx : rbnull;
+            const int sa = (in ? s : 0) * kStepBytes, sb = (in ? s : 0) * 192 * 16;
+            u32x4* d = bs + slot * kPfSlot3;
+#pragma unroll
+            for (int i = 0; i < kPfAPerWave; ++i)
+                load_lds12(ra, d + (wave * kPfAPerWave + i) * 64, aoff[i], sa);
+#pragma unroll
+            for (int j = 0; j < 3; ++j)
+                load_lds16(rb, d + kPfSlotA + wave * 64 + j * kPfThreads, boff3[j], sb);
+        };
+        // steps 0 .. 3 into slots 0 .. 3, then per step: its loads landed,
+        // barrier, its fragments and 48 MFMAs, barrier, the step 4 ahead
+        // into its slot.
+#pragma unroll
+        for (int i = 0; i < kPfRing3; ++i) load_step(i, i);
+        int slot = 0;
+        for (int s = 0; s < s_hi - s_lo; ++s) {
             asm volatile("" ::: "memory");
-            __builtin_amdgcn_s_waitcnt(waitcnt_vm_lgkm0(kPfWait));
+            __builtin_amdgcn_s_waitcnt(waitcnt_vm(kPfWait3));
             __builtin_amdgcn_s_barrier();
             asm volatile("" ::: "memory");
-            load_step(u, s + kPfRing);
-            read_frags(fa[(u + 1) & 1], fb[(u + 1) & 1], (u + 1) % kPfRing);
-            // the reads are issued here, ahead of the MFMAs they overlap
-            asm volatile("" ::: "memory");
-            __builtin_amdgcn_sched_barrier(0);
+            const u32x4* d = bs + slot * kPfSlot3;
             u32x4 a[kPfWB];
 #pragma unroll
             for (int b = 0; b < kPfWB; ++b) {
+                const u32x3 r = *reinterpret_cast<const u32x3*>(d + (wr * kPfWB + b) * 64 + lane);
                 uint32_t pr[4];
-                unpack_pairs(fa[u & 1][b].x, fa[u & 1][b].y, fa[u & 1][b].z, pr);
+                unpack_pairs(r.x, r.y, r.z, pr);
                 a[b] = u32x4{pr[0], pr[1], pr[2], pr[3]};
             }
+            const u32x4* src = d + kPfSlotA + wc * kPfWT * 192 + lane;
 #pragma unroll
             for (int q = 0; q < 3; ++q)
 #pragma unroll
-                for (int b = 0; b < kPfWB; ++b)
+                for (int c = 0; c < kPfWT; ++c) {
+                    const u32x4 bf = src[c * 192 + q * 64];
 #pragma unroll
-                    for (int c = 0; c < kPfWT; ++c) acc[b][c] = mfma(a[b], fb[u & 1][q][c], acc[b][c]);
+                    for (int b = 0; b < kPfWB; ++b) acc[b][c] = mfma(a[b], bf, acc[b][c]);
+                }
+            asm volatile("" ::: "memory");
+            __builtin_amdgcn_s_waitcnt(waitcnt_lgkm0());
+            __builtin_amdgcn_s_barrier();
+            asm volatile("" ::: "memory");
+            load_step(slot, s + kPfRing3);
+            slot = slot + 1 == kPfRing3 ? 0 : slot + 1;
         }
     }
     // the last loads (zeros into slots nobody reads) land before the
@@ -338,169 +496,197 @@ __global__ __launch_bounds__(kPfThreads) void k_prefill_mm(const uint32_t* __res
     asm volatile("" ::: "memory");
     __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));
 
-    // epilogue: lane l holds token 16 c + l%16 and rows 4(l/16) + 0..3 of each tile
+    // epilogue: lane l holds token 16 c + l%16 and rows 4(l/16) + 0..3 of each
+    // tile.  v = acc 2^(sc_row - P_t) (exact), plus the row's exceptions, times
+    // rs with RMS, stored or added; with a K split the split's sums go to
+    // part[sp][token][row] instead (rs and the store or add are the reduce
+    // pass's).  Loads that depend on nothing are issued together ahead of their
+    // use, and four rows of a token are one 16-byte load or store where
+    // N % 4 == 0 (indexes clamped into the matrix instead of branches; what is
+    // read past an edge is not stored): with a load, branch and store per value
+    // the pass took about 20 us of a workgroup, longer than 8 K steps.
     const int q = lane >> 4, jj = lane & 15;
-    // (a) rescale: v = acc 2^(sc_row - P_t), exact
-    float v[kPfWB][kPfWT][4];
-    int tok[kPfWT];
+    const int64_t rlo = blk0 * 16;
+    __builtin_amdgcn_s_barrier();  // the ring's LDS is the exception sums' from here
+    asm volatile("" ::: "memory");
+    if (rlo >= N) return;
+    const int32_t e_lo = rp[rlo], e_hi = rp[min(rlo + 16 * kPfWB, (int64_t)N)];
+    const bool vec = (N & 3) == 0;  // y, part and rbase are 16-byte aligned
+    int64_t nr[kPfWB];              // the lane's first row of each tile
+    int sc[kPfWB][4];
 #pragma unroll
-    for (int c = 0; c < kPfWT; ++c) {
-        tok[c] = (tb0 + wc * kPfWT + c) * 16 + jj;
-        const int pt = tok[c] < T ? P[tok[c]] : 0;
+    for (int b = 0; b < kPfWB; ++b) {
+        nr[b] = rlo + b * 16 + q * 4;
+        if (vec) {
+            const int4 r = *reinterpret_cast<const int4*>(rbase + min(nr[b], (int64_t)N - 4));
+            sc[b][0] = r.x, sc[b][1] = r.y, sc[b][2] = r.z, sc[b][3] = r.w;
+        } else {
 #pragma unroll
-        for (int b = 0; b < kPfWB; ++b) {
-            const int64_t n = (blk0 + b) * 16 + q * 4;
-            const float av[4] = {acc[b][c].x, acc[b][c].y, acc[b][c].z, acc[b][c].w};
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-                v[b][c][i] = ldexpf(av[i], scale_exp(rbase[min(n + i, (int64_t)N - 1)]) - pt);
+            for (int i = 0; i < 4; ++i) sc[b][i] = rbase[min(nr[b] + i, (int64_t)N - 1)];
         }
     }
-    // (b) the exceptions of the wave's 64 rows (the tiles hold zeros there), in
-    // list order, 8 entries at a time, the next batch's metadata and x'
-    // gathers issued before the current one is added: each entry's row,
-    // column and value are wave-uniform (scalar loads), x' of the lane's 4
-    // tokens at its column comes from the transposed copy (the wave's 64
-    // tokens of one column: 256 contiguous bytes), and a switch on the row's
-    // (row block, row) slot adds the product to that output only, in the
-    // lanes of the row's quarter
-    const int64_t rlo = blk0 * 16;
-    if (rlo < N) {
-        const int32_t e_lo = rp[rlo], e_hi = rp[min(rlo + 16 * kPfWB, (int64_t)N)];
+    float* xs = reinterpret_cast<float*>(bs) + wave * (16 * kPfWB * kPfExcStride);  // the wave's [64 rows][64 tokens]
+    const int tbw = tb0 + wc * kPfWT;  // the wave's token blocks
+    // (a) v = acc 2^(sc_row - P_t), exact
+#pragma unroll
+    for (int c = 0; c < kPfWT; ++c) {
+        const int et = E[min((tbw + c) * 16 + jj, T - 1)];
+        const int pt = wide ? scale_bf16(et) : scale_f16(et) + kF16WeightExp;
+#pragma unroll
+        for (int b = 0; b < kPfWB; ++b)
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                acc[b][c][i] = ldexpf(acc[b][c][i], scale_exp(sc[b][i]) - pt);
+    }
+    // (b) the exceptions of the wave's 64 rows (the tiles hold zeros
+    // there) added in list order, lane = token: the sums go through LDS, an
+    // entry's row, column and value are wave-uniform (scalar loads), x' of
+    // the 64 tokens at its column is 256 contiguous bytes of the transposed
+    // copy, and a row's sums stay in a register from its first entry to its
+    // last.  (With a K split, the entries whose column lies in the split's
+    // steps.)  One wave's LDS accesses stay in order; the fences keep the
+    // compiler's in theirs.
+    if (e_lo < e_hi) {
         constexpr int EB = 8;
-        const float* xtw = xt + (int64_t)(tb0 + wc * kPfWT) * 16 + jj;  // token block c at + 16 c
-        // (with a K split, the entries whose column lies in the split's steps)
+#pragma unroll
+        for (int b = 0; b < kPfWB; ++b)
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int c = 0; c < kPfWT; ++c)
+                    xs[(b * 16 + q * 4 + i) * kPfExcStride + c * 16 + jj] = acc[b][c][i];
+        asm volatile("" ::: "memory");
+        const float* xtw = xt + (int64_t)tbw * 16 + lane;
         const int c_lo = s_lo * 32, c_hi = s_hi * 32;
-        int nr[EB];
-        bool nin[EB];
-        float nv[EB], ng[EB][kPfWT];
-        auto fetch = [&](int32_t e0) {
+        int row = 0;
+        float sum = xs[lane];
+        for (int32_t e0 = e_lo; e0 < e_hi; e0 += EB) {
+            int r[EB];
+            float g[EB], v[EB];
 #pragma unroll
             for (int j = 0; j < EB; ++j) {
                 const int32_t e = min(e0 + j, e_hi - 1);
-                nr[j] = (int)(er[e] - rlo);
-                nv[j] = ev[e];
                 const int col = ec[e];
-                nin[j] = col >= c_lo && col < c_hi;
-                const float* xc = xtw + (int64_t)col * tp;
-#pragma unroll
-                for (int c = 0; c < kPfWT; ++c) ng[j][c] = xc[c * 16];
+                const bool in = e0 + j < e_hi && col >= c_lo && col < c_hi;
+                r[j] = in ? (int)(er[e] - rlo) : -1;
+                v[j] = ev[e];
+                g[j] = xtw[(int64_t)col * tp];
             }
-        };
-        // no entry for these rows (n_exc = 0 included, where er / ec / ev may
-        // be null): nothing is fetched, so no index below e_lo is formed
-        if (e_lo < e_hi) fetch(e_lo);
-        for (int32_t e0 = e_lo; e0 < e_hi; e0 += EB) {
-            int rr[EB];
-            bool rin[EB];
-            float evv[EB], xv[EB][kPfWT];
 #pragma unroll
             for (int j = 0; j < EB; ++j) {
-                rr[j] = nr[j];
-                rin[j] = nin[j];
-                evv[j] = nv[j];
-#pragma unroll
-                for (int c = 0; c < kPfWT; ++c) xv[j][c] = ng[j][c];
-            }
-            if (e0 + EB < e_hi) fetch(e0 + EB);
-#pragma unroll
-            for (int j = 0; j < EB; ++j) {
-                if (e0 + j >= e_hi) break;
-                if (!rin[j]) continue;
-                const int r = rr[j];
-                const bool mine = q == ((r & 15) >> 2);
-#define RV12_EXC_CASE(B, I)                                                                 \
-    case (B) * 4 + (I):                                                                     \
-        if (mine) {                                                                         \
-            _Pragma("unroll") for (int c = 0; c < kPfWT; ++c) v[B][c][I] += evv[j] * xv[j][c]; \
-        }                                                                                   \
-        break;
-                static_assert(kPfWB == 4, "one case per (row block, row) slot of the wave");
-                switch (((r >> 4) << 2) | (r & 3)) {
-                    RV12_EXC_CASE(0, 0) RV12_EXC_CASE(0, 1) RV12_EXC_CASE(0, 2) RV12_EXC_CASE(0, 3)
-                    RV12_EXC_CASE(1, 0) RV12_EXC_CASE(1, 1) RV12_EXC_CASE(1, 2) RV12_EXC_CASE(1, 3)
-                    RV12_EXC_CASE(2, 0) RV12_EXC_CASE(2, 1) RV12_EXC_CASE(2, 2) RV12_EXC_CASE(2, 3)
-                    RV12_EXC_CASE(3, 0) RV12_EXC_CASE(3, 1) RV12_EXC_CASE(3, 2) RV12_EXC_CASE(3, 3)
-                    default: break;
+                if (r[j] < 0) continue;
+                if (r[j] != row) {
+                    xs[row * kPfExcStride + lane] = sum;
+                    row = r[j];
+                    sum = xs[row * kPfExcStride + lane];
                 }
-#undef RV12_EXC_CASE
+                sum += v[j] * g[j];
             }
         }
+        xs[row * kPfExcStride + lane] = sum;
+        asm volatile("" ::: "memory");
+#pragma unroll
+        for (int b = 0; b < kPfWB; ++b)
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int c = 0; c < kPfWT; ++c)
+                    acc[b][c][i] = xs[(b * 16 + q * 4 + i) * kPfExcStride + c * 16 + jj];
     }
-    // (c) with RMS the token's rs; store or add; rows past N and tokens past
-    // T are skipped.  With a K split: the split's sums to part[sp][token][row]
-    // (rs and the store or add are the reduce pass's)
-    if (S > 1) {
-        float* ps = part + (int64_t)sp * tp * N;
+    // (c) the outputs
+    int tok[kPfWT];
+    float rs[kPfWT];
+    f32x4 oy[kPfWB][kPfWT];
 #pragma unroll
-        for (int c = 0; c < kPfWT; ++c) {
-            if (tok[c] >= T) continue;
+    for (int c = 0; c < kPfWT; ++c) {
+        tok[c] = (tbw + c) * 16 + jj;
+        const int tc = min(tok[c], T - 1);
+        rs[c] = LN && S == 1 ? R[tc] : 1.0f;
+        const float* yr = y + (int64_t)tc * N;
 #pragma unroll
-            for (int b = 0; b < kPfWB; ++b) {
-                const int64_t n = (blk0 + b) * 16 + q * 4;
+        for (int b = 0; b < kPfWB; ++b) {
+            oy[b][c] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+            if (add && S == 1) {
+                if (vec) {
+                    oy[b][c] = *reinterpret_cast<const f32x4*>(yr + min(nr[b], (int64_t)N - 4));
+                } else {
 #pragma unroll
-                for (int i = 0; i < 4; ++i)
-                    if (n + i < N) ps[(int64_t)tok[c] * N + n + i] = v[b][c][i];
+                    for (int i = 0; i < 4; ++i) oy[b][c][i] = yr[min(nr[b] + i, (int64_t)N - 1)];
+                }
             }
         }
-        return;
     }
 #pragma unroll
     for (int c = 0; c < kPfWT; ++c) {
-        if (tok[c] >= T) continue;
-        if constexpr (LN) {
-            const float rs = R[tok[c]];
-#pragma unroll
-            for (int b = 0; b < kPfWB; ++b)
-#pragma unroll
-                for (int i = 0; i < 4; ++i) v[b][c][i] *= rs;
-        }
+        float* dst = S > 1 ? part + ((int64_t)sp * tp + tok[c]) * N : y + (int64_t)tok[c] * N;
 #pragma unroll
         for (int b = 0; b < kPfWB; ++b) {
-            const int64_t n = (blk0 + b) * 16 + q * 4;
+            f32x4 v = acc[b][c];
+            if constexpr (LN) v *= rs[c];
+            if (add && S == 1) v = oy[b][c] + v;
+            if (tok[c] >= T) continue;
+            if (vec) {
+                if (nr[b] < N) *reinterpret_cast<f32x4*>(dst + nr[b]) = v;
+            } else {
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                if (n + i >= N) continue;
-                float* yp = y + (int64_t)tok[c] * N + n + i;
-                *yp = add ? *yp + v[b][c][i] : v[b][c][i];
+                for (int i = 0; i < 4; ++i)
+                    if (nr[b] + i < N) dst[nr[b] + i] = v[i];
             }
         }
     }
 }
 
-int prefill_tokens_padded(int T) { return (T + kPfTokBlocks * 16 - 1) / (kPfTokBlocks * 16) * (kPfTokBlocks * 16); }
+int prefill_tokens_padded(int T) { return (T + kPfTokens - 1) / kPfTokens * kPfTokens; }
 
-// 3. (K split only) y[t][n] (=|+=) rs_t * sum over the splits, in split order
+// 3. (K split only) y[t][n] (=|+=) rs_t * sum over the splits, in split order:
+// V consecutive rows per thread (4 where N % 4 == 0), the loads of 4 splits and
+// the old y in flight together
+template <int V>
 __global__ __launch_bounds__(256) void k_prefill_reduce(const float* __restrict__ part, const float* __restrict__ R,
                                                         float* __restrict__ y, int64_t N, int T, int tp, int S,
                                                         int add) {
-    const int64_t n = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    typedef float fv __attribute__((ext_vector_type(V)));
+    const int64_t n = ((int64_t)blockIdx.x * 256 + threadIdx.x) * V;
     if (n >= N) return;
     for (int t = blockIdx.y; t < T; t += gridDim.y) {
-        float v = 0.0f;
-        for (int sp = 0; sp < S; ++sp) v += part[((int64_t)sp * tp + t) * N + n];
-        if (R) v *= R[t];
         float* yp = y + (int64_t)t * N + n;
-        *yp = add ? *yp + v : v;
+        const float* ps = part + (int64_t)t * N + n;
+        const int64_t step = (int64_t)tp * N;
+        const float rs = R ? R[t] : 1.0f;
+        fv old = {}, v = {};
+        if (add) old = *reinterpret_cast<const fv*>(yp);
+        for (int sp = 0; sp < S; sp += 4) {
+            fv a[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) a[u] = *reinterpret_cast<const fv*>(ps + min(sp + u, S - 1) * step);
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+                if (sp + u < S) v += a[u];
+        }
+        if (R) v *= rs;
+        *reinterpret_cast<fv*>(yp) = add ? old + v : v;
     }
 }
 
-// K splits of the GEMM: the fewest that minimise a model of its rounds of
-// workgroups (one per CU) — each round costs the steps of a split at 1.4 us
-// plus 10 us — and of the reduce pass over the (S + 1) T N partial floats
-// (3 us + bytes at 5 TB/s); no split below 8 steps
+// K splits of the GEMM: those of the least modelled time.  A round of
+// workgroups (one per CU) costs its steps plus 8 us of prologue and epilogue, a
+// step 0.8 us and up to 0.2 more as the chip fills (its clock falls); the
+// reduce pass costs 4 us + (S + 1) T N floats at 5 TB/s (1024 x 3072 over 301
+// tokens: 92 us unsplit, 36 with 12 splits; 4096 x 4096 over 2048, one full
+// round: 160 unsplit, 183 with 2).  No split below 8 steps.
 int prefill_splits(int N, int K, int T) {
     const int64_t nx = ((int64_t)N + 16 * kPfRowBlocks - 1) / (16 * kPfRowBlocks);
-    const int64_t tp = prefill_tokens_padded(T);
-    const int64_t G = nx * (tp / (kPfTokBlocks * 16));
-    const int nsteps = K / 32;
+    const int tp = prefill_tokens_padded(T), nsteps = K / 32;
+    const int64_t G = nx * (tp / kPfTokens);
     int best = 1;
     double best_us = 0.0;
     for (int S = 1; S <= 16; ++S) {
         if (S > 1 && nsteps / S < 8) break;
-        const double rounds = (double)((G * S + 255) / 256);
-        double us = rounds * ((double)nsteps / S * 1.4 + 10.0);
-        if (S > 1) us += 3.0 + (double)(S + 1) * tp * N * 4 / 5e6;
+        const double steps = (nsteps + S - 1) / S;
+        const double last = (double)(G * S % 256) / 256;
+        double us = (double)(G * S / 256) * (steps * 1.0 + 8.0);
+        if (last > 0) us += steps * (0.8 + 0.2 * last * last) + 8.0;
+        if (S > 1) us += 4.0 + (double)(S + 1) * tp * N * 4 / 5e6;
         if (S == 1 || us < best_us) {
             best = S;
             best_us = us;
@@ -512,7 +698,7 @@ int prefill_splits(int N, int K, int T) {
 size_t prefill_ws_bytes(int N, int K, int T) {
     const size_t tp = (size_t)prefill_tokens_padded(T);
     const int S = prefill_splits(N, K, T);
-    // parts, P and R, transposed x', split partials
+    // parts (room for three), E and R, transposed x', split partials
     return tp * (size_t)K * 10 + tp * 8 + (S > 1 ? (size_t)S * tp * (size_t)N * 4 : 0);
 }
 
@@ -521,27 +707,30 @@ void launch_prefill(const rv12_matrix& w, const float* x, float* y, int T, int m
     const int K = w.k, N = w.n;
     const int tp = prefill_tokens_padded(T);
     u32x4* xb = reinterpret_cast<u32x4*>(ws);
-    int* P = reinterpret_cast<int*>(reinterpret_cast<char*>(ws) + (size_t)tp * K * 6);
-    float* R = reinterpret_cast<float*>(P + tp);
+    int* E = reinterpret_cast<int*>(reinterpret_cast<char*>(ws) + (size_t)tp * K * 6);
+    float* R = reinterpret_cast<float*>(E + tp);
     float* xt = R + tp;
     float* part = xt + (size_t)tp * K;
     const int xs = mode == 2 ? 2 * K : K;
     const int m2 = mode == 2 ? 1 : 0;
-    hipLaunchKernelGGL(k_prefill_stats, dim3(tp / (kPsThreads / 64)), dim3(kPsThreads), 0, st, x, T, K, xs, m2, lnw, eps,
-                       P, R);
-    hipLaunchKernelGGL(k_prefill_parts, dim3(tp / 32, (K + 63) / 64), dim3(kPpThreads), 0, st, x, T, K, xs, m2, lnw, P,
-                       xb, xt, tp);
     const int S = prefill_splits(N, K, T);
+    hipLaunchKernelGGL(k_prefill_stats, dim3(tp / (kPsThreads / 64)), dim3(kPsThreads), 0, st, x, T, K, xs, m2, lnw, eps,
+                       E, R);
+    hipLaunchKernelGGL(k_prefill_parts, dim3(tp / 32, (K + 63) / 64), dim3(kPpThreads), 0, st, x, T, K, xs, m2, lnw, E,
+                       xb, xt, tp);
     const int64_t nblk = ((int64_t)N + 15) / 16;
-    const dim3 grid((unsigned)((nblk + kPfRowBlocks - 1) / kPfRowBlocks * (tp / (kPfTokBlocks * 16))), (unsigned)S);
+    const dim3 grid((unsigned)((nblk + kPfRowBlocks - 1) / kPfRowBlocks * (tp / kPfTokens)), (unsigned)S);
     const auto kern = lnw ? k_prefill_mm<true> : k_prefill_mm<false>;
     (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
                               (int)kPfLds);
     hipLaunchKernelGGL(kern, grid, dim3(kPfThreads), kPfLds, st, reinterpret_cast<const uint32_t*>(w.tiles), w.rbase, xb,
-                       P, w.rp, w.er, w.ec, w.ev, xt, tp, R, y, part, N, K, T, mode != 0 ? 1 : 0);
-    if (S > 1)
-        hipLaunchKernelGGL(k_prefill_reduce, dim3((unsigned)((N + 255) / 256), (unsigned)min(T, 65535)), dim3(256), 0, st, part,
+                       E, w.rp, w.er, w.ec, w.ev, xt, tp, R, y, part, N, K, T, mode != 0 ? 1 : 0);
+    if (S > 1) {
+        const int V = N % 4 == 0 ? 4 : 1;
+        const dim3 rgrid((unsigned)((N + 256 * V - 1) / (256 * V)), (unsigned)min(T, 65535));
+        hipLaunchKernelGGL((V == 4 ? k_prefill_reduce<4> : k_prefill_reduce<1>), rgrid, dim3(256), 0, st, part,
                            lnw ? R : nullptr, y, (int64_t)N, T, tp, S, mode != 0 ? 1 : 0);
+    }
 }
 
 }  // namespace rv12

@@ -228,10 +228,12 @@ int rv12_gemm_static(const rv12_matrix* w, const float* x, float* y, int t, cons
 /* The prompt's linear, 1 <= t <= 65536 tokens at once:  y[r] (=|+=) W_dec . x'[r]
  * for every token row r (x rows K floats apart, 2K in mode 2; y rows N apart),
  * mode and lnw / eps (the RMSNorm prologue, modes 0 and 1; 16-byte aligned)
- * as rv12_gemv.  The 12-bit decode is fused into a bf16 MFMA GEMM:
- * x' is split per token into three bf16 parts (24 significand bits, after an
- * exact power-of-two scale), every weight is read once in its 12-bit form,
- * products and sums are fp32, the exceptions are added in list order.  Where
+ * as rv12_gemv.  The 12-bit decode is fused into an MFMA GEMM:
+ * x' is split per token into two float16 parts (22 significand bits, after an
+ * exact power-of-two scale), or into three bf16 parts (24 bits) in a tile of
+ * tokens one of which spreads over more exponents than float16 holds; every
+ * weight is read once in its 12-bit form, products and sums are fp32, the
+ * exceptions are added in list order.  Where
  * the rows and tokens give too few workgroups to fill the GPU (few tokens, or
  * a last round of workgroups mostly empty), K is split and an ordered pass
  * sums the splits.  ws: rv12_prefill_workspace_bytes(n, k, t) bytes (10 bytes

@@ -227,3 +227,46 @@ def test_matrix_on_golden_special_values(golden, case):
     cnp = ref_dict(golden[case])
     for add in (False, True):
         _check(cnp, 40, 3, add)
+
+
+@pytest.mark.parametrize("K", [512, 544, 1056])
+@pytest.mark.parametrize("T", [300, 513])
+def test_unsplit_sums_over_chunks_of_steps(K, T):
+    """Enough rows for unsplit workgroups whose K steps are a whole chunk of the
+    fp32 sums, one step more, and two chunks and one step; rows off the vector
+    store's four, one token in the last tile."""
+    rng = np.random.default_rng(K + T)
+    N = 22003
+    w = (rng.standard_normal((N, K)) * 0.02).astype(np.float32)
+    w[rng.choice(N, 20, replace=False)] *= 20
+    w.reshape(-1)[rng.choice(w.size, 300, replace=False)] = 1e-30
+    cnp = codec.compress(codec.f32_to_bf16_rne(w), CH=32)
+    for mode, rms in ((0, True), (1, False)):
+        print("K", K, "T", T, "mode", mode, "rms", rms, flush=True)
+        _check(cnp, T, K + T + mode, mode != 0, mode=mode, rms=rms)
+
+
+@pytest.mark.parametrize("N,T", [(300, 300), (22003, 300)])
+@pytest.mark.parametrize("big", [0, 20, 40])
+def test_tokens_over_many_exponents(N, T, big):
+    """Values 2^big above the rest in a column whose weights are zero: the
+    output is the other columns' alone, and the fp32 bound of those alone holds,
+    which float16 parts scaled to the huge value would miss by far.  Tiles with
+    and without such a token, split and unsplit."""
+    from ai_amd import prefill, wcomp
+    rng = np.random.default_rng(big)
+    K = 256
+    w = (rng.standard_normal((N, K)) * 0.02).astype(np.float32)
+    w[:, 77] = 0
+    bits = codec.f32_to_bf16_rne(w)
+    x = rng.standard_normal((T, K)).astype(np.float32)
+    x[[3, 5, T - 1]] *= np.float32(2.0) ** -big
+    x[[3, 5, T - 1], 77] = 1.5
+    c = wcomp.compress(torch.from_numpy(bits.view(np.int16)).view(torch.bfloat16).cuda())
+    y = torch.zeros(T, N, device="cuda")
+    prefill.matrix(torch.from_numpy(x).cuda(), c, y)
+    w64 = codec.bf16_to_f32(bits).astype(np.float64)
+    w64[:, 77] = 0
+    want, mag = x.astype(np.float64) @ w64.T, np.abs(x.astype(np.float64)) @ np.abs(w64).T
+    err = np.abs(y.cpu().numpy() - want)
+    assert np.all(err <= 4 * (K + 8) * 2.0 ** -24 * mag + 1e-30), float((err / mag).max())
