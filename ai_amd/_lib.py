@@ -27,7 +27,8 @@ EXPORTS = ("rv12_abi_version", "rv12_strerror", "rv12_tiles_bytes", "rv12_pack_p
            "rv12_gemv", "rv12_gemm", "rv12_gemm_static", "rv12_decode_rows", "rv12_attn_workspace_bytes", "rv12_rope_attn",
            "rv12_attn_batch_workspace_bytes", "rv12_rope_attn_batch", "rv12_prefill_attn_workspace_bytes",
            "rv12_prefill_rope_attn", "rv12_prefill_workspace_bytes",
-           "rv12_prefill_linear", "rv12_decode_advance")
+           "rv12_prefill_linear", "rv12_decode_advance",
+           "rv12_compress_workspace_bytes", "rv12_compress_plan", "rv12_compress_write")
 ABI_VERSION = 8
 STATIC_SCRATCH_BYTES = 8 << 20  # RV12_STATIC_SCRATCH_BYTES
 
@@ -97,6 +98,12 @@ def lib():
         L.rv12_encode.argtypes = [P, I, I, I, I, P, P, P, P]
         L.rv12_encode_exc.restype = I
         L.rv12_encode_exc.argtypes = [P, I, I, I, P, P, P, P, P]
+        L.rv12_compress_workspace_bytes.restype = SZ
+        L.rv12_compress_workspace_bytes.argtypes = [I, I]
+        L.rv12_compress_plan.restype = I
+        L.rv12_compress_plan.argtypes = [P, I, I, P, P, P, P, P, SZ, P]
+        L.rv12_compress_write.restype = I
+        L.rv12_compress_write.argtypes = [P, I, I, I, P, I64, P, P, P, P, P, I64, P, SZ, P, P, P, P]
         L.rv12_launch_shape.restype = I
         L.rv12_launch_shape.argtypes = [I, I, I, ctypes.POINTER(Launch), ctypes.POINTER(Launch)]
         L.rv12_workspace_bytes.restype = SZ

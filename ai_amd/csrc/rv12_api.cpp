@@ -444,6 +444,33 @@ int rv12_encode_exc(const uint16_t* w, int n, int k, int base, const int32_t* rp
     return launch_status();
 }
 
+size_t rv12_compress_workspace_bytes(int n, int k) { return shape_ok(n, k) ? compress_ws_bytes(n) : 0; }
+
+int rv12_compress_plan(const uint16_t* w, int n, int k, int32_t* rbase, int32_t* rp, int32_t* qrp, int32_t* out,
+                       void* ws, size_t ws_bytes, void* stream) {
+    if (!w || !rbase || !rp || !qrp || !out) return RV12_E_NULL;
+    if (!shape_ok(n, k)) return RV12_E_SHAPE;
+    if (!ws || ws_bytes < compress_ws_bytes(n)) return RV12_E_WORKSPACE;
+    if (!aligned16(w) || !aligned16(ws)) return RV12_E_ALIGN;
+    launch_compress_plan(w, n, k, rbase, rp, qrp, out, ws, (hipStream_t)stream);
+    return launch_status();
+}
+
+int rv12_compress_write(const uint16_t* w, int n, int k, int base, const int32_t* rp, int64_t n_exc, int32_t* er,
+                        int32_t* ec, float* ev, const int32_t* rbase, const int32_t* qrp, int64_t n_qexc,
+                        uint32_t* tiles, size_t tiles_bytes, int32_t* qer, int32_t* qec, float* qev, void* stream) {
+    if (!w || !rp || !rbase || !qrp || !tiles) return RV12_E_NULL;
+    if (n_exc > 0 && (!er || !ec || !ev)) return RV12_E_NULL;
+    if (n_qexc > 0 && (!qer || !qec || !qev)) return RV12_E_NULL;
+    if (!shape_ok(n, k) || n_exc < 0 || n_qexc < 0) return RV12_E_SHAPE;
+    if (base < 0 || base > 241) return RV12_E_BASE;
+    if (!aligned16(w) || !aligned16(tiles)) return RV12_E_ALIGN;
+    if (tiles_bytes < rv12_tiles_bytes(n, k)) return RV12_E_SIZE;
+    launch_compress_write(w, n, k, base, rp, er, ec, ev, n_exc, rbase, qrp, qer, qec, qev, n_qexc, tiles,
+                          (hipStream_t)stream);
+    return launch_status();
+}
+
 int rv12_launch_shape(int n, int k, int t, const rv12_launch* cfg, rv12_launch* out) {
     if (!out) return RV12_E_NULL;
     if (n < 1 || k < 32 || k % 32 || k > kMaxK) return RV12_E_SHAPE;

@@ -1,11 +1,16 @@
 // rv12 codec kernels for gfx950.
 //   encode   the reference 12-bit codec dict of a bf16 matrix: exponent
 //            histogram, m8/e4, row-major exception list (k_hist,
-//            k_encode_rows, k_encode_exc)
+//            k_encode_rows, k_exceptions)
 //   to_bf16  a codec dict back to bf16 bits (k_codec_to_bf16 + k_scatter_exc)
 //   pack     bf16 bits -> the Q16 layout with one exponent window per row and
-//            that layout's own exception list (k_row_base, k_pack_count,
-//            k_pack_tiles, k_encode_exc)
+//            that layout's own exception list (k_row_windows, k_pack_tiles,
+//            k_exceptions)
+//   compress the packed form and the reference codec's base, row pointers and
+//            exception list together (k_row_windows, k_hist_sum, k_row_counts,
+//            k_row_pointers, k_pack_tiles, k_exceptions with both lists): two
+//            reads of the weights, a third of the rows with entries, one host
+//            read between (6144 x 4096: 79 us, 377 as separate calls)
 //   decode   Q16 rows back to the exact bf16 / float32 values (k_decode,
 //            k_decode_exc)
 // The Q16 layout and the h encoding are described in rv12_device.h.
@@ -77,47 +82,92 @@ __global__ __launch_bounds__(256) void k_encode_rows(const uint16_t* __restrict_
     }
 }
 
-// one workgroup per row: exceptions in column order at rp[n]
-// (base = rbase[n] when rbase is given: the row windows of the packed form)
-__global__ __launch_bounds__(256) void k_encode_exc(const uint16_t* __restrict__ w, int K, int base,
-                                                    const int32_t* __restrict__ rbase,
-                                                    const int32_t* __restrict__ rp, int32_t* __restrict__ er,
-                                                    int32_t* __restrict__ ec, float* __restrict__ ev) {
-    const int n = blockIdx.x;
-    if (rbase) base = rbase[n];
-    const int32_t start = rp[n];
-    if (rp[n + 1] == start) return;  // uniform across the workgroup
+// One list of weights outside an exponent window: the window start of row n is
+// rbase[n], or base where rbase is null; the row's entries go to rp[n] on.
+struct ExcList {
+    const int32_t* rbase;
+    int base;
+    const int32_t* rp;
+    int32_t* er;
+    int32_t* ec;
+    float* ev;
+};
+
+// One wave per row, up to two lists at once (the codec's and the packed form's):
+// a row without entries is not read; otherwise lane l takes 8 consecutive
+// weights of each 512, four such chunks in flight, and a chunk without entries
+// (nearly all) costs one ballot.  In a chunk with some, a wave scan of the
+// lanes' counts gives their places in column order.  Bound by reading the rows
+// that have entries (6144 x 4096, one entry in 6553 weights: 13 us for both
+// lists, 64 for each with a thread per 16 consecutive weights).
+// VEC: K % 8 == 0 and w 16-byte aligned.
+constexpr int kExcWaves = 4;
+template <bool VEC>
+__global__ __launch_bounds__(kExcWaves * 64) void k_exceptions(const uint16_t* __restrict__ w, int N, int K, ExcList a,
+                                                               ExcList b, int nlists) {
+    const int lane = threadIdx.x & 63;
+    const int n = blockIdx.x * kExcWaves + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if (n >= N) return;
+    int posa = a.rp[n], posb = nlists > 1 ? b.rp[n] : 0;
+    const bool ina = a.rp[n + 1] != posa, inb = nlists > 1 && b.rp[n + 1] != posb;
+    if (!ina && !inb) return;
+    const int basea = a.rbase ? a.rbase[n] : a.base, baseb = nlists > 1 ? (b.rbase ? b.rbase[n] : b.base) : 0;
     const uint16_t* row = w + (int64_t)n * K;
-    const int per = (K + blockDim.x - 1) / blockDim.x;
-    const int k0 = threadIdx.x * per, k1 = min(K, k0 + per);
-    int cnt = 0;
-    for (int k = k0; k < k1; ++k) {
-        int c = (int)((row[k] >> 7) & 0xFF) - base;
-        cnt += (c < 0 || c > 14);
-    }
-    // exclusive scan of cnt over the workgroup
-    __shared__ int wsum[4];
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    int inc = cnt;
-    for (int d = 1; d < 64; d <<= 1) {
-        int v = __shfl_up(inc, d);
-        if (lane >= d) inc += v;
-    }
-    if (lane == 63) wsum[wv] = inc;
-    __syncthreads();
-    int off = inc - cnt;
-    for (int i = 0; i < wv; ++i) off += wsum[i];
-    int pos = start + off;
-    for (int k = k0; k < k1; ++k) {
-        uint32_t b = row[k];
-        int c = (int)((b >> 7) & 0xFF) - base;
-        if (c < 0 || c > 14) {
-            er[pos] = n;
-            ec[pos] = k;
-            ev[pos] = __uint_as_float(b << 16);
-            ++pos;
+    auto put = [&](const ExcList& l, int& pos, uint32_t mask, const uint32_t (&bits)[4], int k) {
+        const int cnt = __popc(mask);
+        int inc = cnt;
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1) {
+            const int v = __shfl_up(inc, d);
+            if (lane >= d) inc += v;
+        }
+        int at = pos + inc - cnt;
+        pos += __shfl(inc, 63);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            if (!(mask >> j & 1)) continue;
+            l.er[at] = n;
+            l.ec[at] = k + j;
+            l.ev[at] = __uint_as_float((j & 1) ? (bits[j >> 1] & 0xFFFF0000u) : (bits[j >> 1] << 16));
+            ++at;
+        }
+    };
+    constexpr int U = 4;
+    for (int k0 = lane * 8; k0 - lane * 8 < K; k0 += 512 * U) {
+        uint32_t d[U][4];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int k = k0 + u * 512;
+            if constexpr (VEC) {
+                const uint4 v = k < K ? *reinterpret_cast<const uint4*>(row + k) : make_uint4(0, 0, 0, 0);
+                d[u][0] = v.x, d[u][1] = v.y, d[u][2] = v.z, d[u][3] = v.w;
+            } else {
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                    d[u][j] = (k + 2 * j < K ? row[k + 2 * j] : 0u) | (k + 2 * j + 1 < K ? row[k + 2 * j + 1] : 0u) << 16;
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int k = k0 + u * 512;
+            uint32_t ma = 0, mb = 0;
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                const int e = (int)((d[u][j >> 1] >> ((j & 1) * 16 + 7)) & 0xFF);
+                const bool in = k + j < K;
+                ma |= (uint32_t)(in && (uint32_t)(e - basea) > 14u) << j;
+                mb |= (uint32_t)(in && (uint32_t)(e - baseb) > 14u) << j;
+            }
+            if (ina && __ballot(ma != 0) != 0) put(a, posa, ma, d[u], k);
+            if (inb && __ballot(mb != 0) != 0) put(b, posb, mb, d[u], k);
         }
     }
+}
+
+static void launch_exceptions(const uint16_t* w, int N, int K, const ExcList& a, const ExcList* b, hipStream_t st) {
+    const bool vec = K % 8 == 0 && reinterpret_cast<uintptr_t>(w) % 16 == 0;
+    hipLaunchKernelGGL((vec ? k_exceptions<true> : k_exceptions<false>), dim3((unsigned)((N + kExcWaves - 1) / kExcWaves)),
+                       dim3(kExcWaves * 64), 0, st, w, N, K, a, b ? *b : a, b ? 2 : 1);
 }
 
 // ------------------------------------------------------------------ to_bf16
@@ -158,64 +208,204 @@ __global__ __launch_bounds__(256) void k_scatter_exc(const int32_t* __restrict__
 }
 
 // ------------------------------------------------------------------ pack
-// one workgroup per row: the row's exponent window, chosen by the reference's
-// rule for a whole matrix (wcomp.py:19-21): the first start b whose 15-wide
-// window [b, b+14] holds the most weights
-__global__ __launch_bounds__(256) void k_row_base(const uint16_t* __restrict__ w, int K, int32_t* __restrict__ rbase) {
-    __shared__ int32_t h[256];
-    __shared__ int32_t win[256];
-    const int64_t n = blockIdx.x;
-    h[threadIdx.x] = 0;
-    __syncthreads();
-    const uint16_t* row = w + n * (int64_t)K;
-    for (int k = threadIdx.x * 8; k < K; k += blockDim.x * 8) {
-        const uint4 v = *reinterpret_cast<const uint4*>(row + k);
+// Every row's exponent window, chosen by the reference's rule for a whole
+// matrix (wcomp.py:19-21): the first start b whose 15-wide window [b, b+14]
+// holds the most weights; rbase[n] = b, row_exc[n] = the weights outside it.
+// One pass over the weights, one wave per row (a grid-stride loop): counts of
+// the 256 exponents in LDS, 16 copies per wave (copy lane % 16, 260 words apart,
+// so that the few exponents most weights have fall on different banks and seldom
+// on the same word); the copies are never cleared: a row's counts are the
+// difference to the wave's running totals, whose sum over the grid is the whole
+// matrix's histogram.  cs (may be null): each row's 256 inclusive prefix counts;
+// part (with cs): the workgroup's share of the histogram.  Bound by the LDS
+// counts beside the read of the weights (6144 x 4096: 15.6 us, 3.2 TB/s, where
+// separate passes for the histogram, windows and counts, with one copy per
+// workgroup, took 53, 60 and 9).
+constexpr int kRowWaves = 4, kRowCopies = 16, kRowPitch = 260;
+constexpr size_t kRowLds = (size_t)kRowWaves * (kRowCopies * kRowPitch + 256) * 4;
+constexpr int kRowGrid = 512;  // two workgroups per CU
+__global__ __launch_bounds__(kRowWaves * 64) void k_row_windows(const uint16_t* __restrict__ w, int N, int K,
+                                                                int32_t* __restrict__ rbase,
+                                                                int32_t* __restrict__ row_exc,
+                                                                int32_t* __restrict__ cs,
+                                                                int32_t* __restrict__ part) {
+    extern __shared__ int32_t lds_i[];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    int32_t* h = lds_i + wave * (kRowCopies * kRowPitch + 256);
+    int32_t* pre = h + kRowCopies * kRowPitch;  // the row's prefix counts
+    for (int i = lane * 4; i < kRowCopies * kRowPitch; i += 256) *reinterpret_cast<int4*>(h + i) = make_int4(0, 0, 0, 0);
+    int32_t* hc = h + (lane % kRowCopies) * kRowPitch;
+    int tot[4] = {0, 0, 0, 0};  // running totals of exponents 4 lane .. 4 lane + 3
+    auto count = [&](uint4 v) {
         const uint32_t d[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-            atomicAdd(&h[(d[j] >> 7) & 0xFF], 1);
-            atomicAdd(&h[(d[j] >> 23) & 0xFF], 1);
+            atomicAdd(&hc[(d[j] >> 7) & 0xFF], 1);
+            atomicAdd(&hc[(d[j] >> 23) & 0xFF], 1);
         }
+    };
+    for (int n = blockIdx.x * kRowWaves + wave; n < N; n += gridDim.x * kRowWaves) {
+        const uint16_t* row = w + (int64_t)n * K;
+        constexpr int U = 4;
+        int k = lane * 8;
+        for (; k + 512 * (U - 1) < K; k += 512 * U) {
+            uint4 v[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) v[u] = *reinterpret_cast<const uint4*>(row + k + u * 512);
+#pragma unroll
+            for (int u = 0; u < U; ++u) count(v[u]);
+        }
+        for (; k < K; k += 512) count(*reinterpret_cast<const uint4*>(row + k));
+        // (one wave's LDS accesses stay in order; the fences keep the compiler's)
+        asm volatile("" ::: "memory");
+        int c[4] = {0, 0, 0, 0};
+#pragma unroll
+        for (int i = 0; i < kRowCopies; ++i) {
+            const int4 q = *reinterpret_cast<const int4*>(h + i * kRowPitch + lane * 4);
+            c[0] += q.x, c[1] += q.y, c[2] += q.z, c[3] += q.w;
+        }
+        int s[4], run = 0;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int r = c[j] - tot[j];
+            tot[j] = c[j];
+            run += r;
+            s[j] = run;
+        }
+        int inc = run;
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1) {
+            const int v = __shfl_up(inc, d);
+            if (lane >= d) inc += v;
+        }
+        const int before = inc - run;  // weights of exponents below 4 lane
+        const int4 ps = make_int4(before + s[0], before + s[1], before + s[2], before + s[3]);
+        *reinterpret_cast<int4*>(pre + lane * 4) = ps;
+        if (cs) *reinterpret_cast<int4*>(cs + (int64_t)n * 256 + lane * 4) = ps;
+        asm volatile("" ::: "memory");
+        int best = -1;  // count * 256 + 255 - b: the largest count, the first b of it (K <= 2^20)
+        const int below[4] = {before, ps.x, ps.y, ps.z};
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int b = lane * 4 + j;
+            if (b <= 241) best = max(best, (pre[b + 14] - below[j]) * 256 + 255 - b);
+        }
+#pragma unroll
+        for (int o = 32; o >= 1; o >>= 1) best = max(best, __shfl_xor(best, o));
+        if (lane == 0) {
+            rbase[n] = 255 - (best & 255);
+            row_exc[n] = K - (best >> 8);
+        }
+        asm volatile("" ::: "memory");
     }
-    __syncthreads();
-    int sum = 0;
-    if (threadIdx.x <= 241)
-        for (int j = 0; j < 15; ++j) sum += h[threadIdx.x + j];
-    win[threadIdx.x] = threadIdx.x <= 241 ? sum : -1;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        int best = 0;
-        for (int j = 1; j <= 241; ++j)
-            if (win[j] > win[best]) best = j;
-        rbase[n] = best;
+    if (part) {
+        *reinterpret_cast<int4*>(pre + lane * 4) = make_int4(tot[0], tot[1], tot[2], tot[3]);
+        __syncthreads();
+        int sum = 0;
+#pragma unroll
+        for (int i = 0; i < kRowWaves; ++i)
+            sum += lds_i[i * (kRowCopies * kRowPitch + 256) + kRowCopies * kRowPitch + threadIdx.x];
+        part[(int64_t)blockIdx.x * 256 + threadIdx.x] = sum;
     }
 }
+static_assert(kRowWaves * 64 == 256 && kRowCopies * kRowPitch % 4 == 0, "one thread per exponent");
 
-// one workgroup per row: weights outside the row's window
-__global__ __launch_bounds__(256) void k_pack_count(const uint16_t* __restrict__ w, int K,
-                                                    const int32_t* __restrict__ rbase,
-                                                    int32_t* __restrict__ row_exc) {
-    const int n = blockIdx.x;
-    const int base = rbase[n];
-    const uint16_t* row = w + (int64_t)n * K;
-    int cnt = 0;
-    for (int k = threadIdx.x * 8; k < K; k += blockDim.x * 8) {
-        const uint4 v = *reinterpret_cast<const uint4*>(row + k);
-        const uint32_t d[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int c0 = (int)((d[j] >> 7) & 0xFF) - base, c1 = (int)((d[j] >> 23) & 0xFF) - base;
-            cnt += (c0 < 0 || c0 > 14) + (c1 < 0 || c1 > 14);
-        }
-    }
-    __shared__ int red[4];
-    for (int o = 32; o > 0; o >>= 1) cnt += __shfl_xor(cnt, o);
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = cnt;
+// The matrix's histogram from the parts, 4 exponents per workgroup (one
+// workgroup over all of them, and over the rows' counts below, waits for one
+// CU's loads: 38 us of a 6144 x 4096 matrix where these passes take about 12).
+constexpr int kHistBins = 4;
+__global__ __launch_bounds__(256) void k_hist_sum(const int32_t* __restrict__ part, int nparts,
+                                                  int64_t* __restrict__ hist) {
+    __shared__ int64_t red[256];
+    const int t = threadIdx.x, bin = blockIdx.x * kHistBins + t % kHistBins;
+    int64_t sum = 0;
+#pragma unroll 8
+    for (int i = t / kHistBins; i < nparts; i += 256 / kHistBins) sum += part[(int64_t)i * 256 + bin];
+    red[t] = sum;
     __syncthreads();
-    if (threadIdx.x == 0) {
-        int t = 0;
-        for (int i = 0; i < (int)(blockDim.x >> 6); ++i) t += red[i];
-        row_exc[n] = t;
+    for (int d = 128; d >= kHistBins; d >>= 1) {
+        if (t < d) red[t] += red[t + d];
+        __syncthreads();
+    }
+    if (t < kHistBins) hist[bin] = red[t];
+}
+
+// The matrix's own window (every workgroup finds it, by the same rule) and each
+// row's weights outside it, from the row's prefix counts.
+__global__ __launch_bounds__(256) void k_row_counts(const int64_t* __restrict__ hist, const int32_t* __restrict__ cs,
+                                                    int N, int K, int32_t* __restrict__ row_exc,
+                                                    int32_t* __restrict__ out) {
+    __shared__ int64_t h[256];
+    __shared__ int64_t red[4];
+    const int t = threadIdx.x;
+    h[t] = hist[t];
+    __syncthreads();
+    int64_t key = -1;  // count * 256 + 255 - b: the largest count, the first b of it
+    if (t <= 241) {
+        int64_t c = 0;
+        for (int j = 0; j < 15; ++j) c += h[t + j];
+        key = c * 256 + 255 - t;
+    }
+#pragma unroll
+    for (int o = 32; o >= 1; o >>= 1) key = max(key, (int64_t)__shfl_xor((long long)key, o));
+    if ((t & 63) == 0) red[t >> 6] = key;
+    __syncthreads();
+    const int base = 255 - (int)(max(max(red[0], red[1]), max(red[2], red[3])) & 255);
+    const int n = blockIdx.x * 256 + t;
+    if (n < N) {
+        const int32_t* r = cs + (int64_t)n * 256;
+        row_exc[n] = K - (r[base + 14] - (base > 0 ? r[base - 1] : 0));
+    }
+    if (n == 0) out[0] = base;
+}
+
+// One workgroup: the row pointers of both exception lists from the rows' counts
+// (16-byte aligned), out = {base (as it is), entries, packed entries}.
+constexpr int kPlanThreads = 1024, kPlanRows = 4 * kPlanThreads;
+__global__ __launch_bounds__(kPlanThreads) void k_row_pointers(const int32_t* __restrict__ exc,
+                                                               const int32_t* __restrict__ qexc, int N,
+                                                               int32_t* __restrict__ rp, int32_t* __restrict__ qrp,
+                                                               int32_t* __restrict__ out) {
+    __shared__ int32_t wsum[2][16];
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    int32_t ca = 0, cb = 0;  // entries of the rows before this tile
+    for (int n0 = 0; n0 < N; n0 += kPlanRows) {
+        const int n = n0 + t * 4;
+        int a[4] = {0, 0, 0, 0}, b[4] = {0, 0, 0, 0};
+        if (n + 3 < N) {
+            const int4 va = *reinterpret_cast<const int4*>(exc + n), vb = *reinterpret_cast<const int4*>(qexc + n);
+            a[0] = va.x, a[1] = va.y, a[2] = va.z, a[3] = va.w;
+            b[0] = vb.x, b[1] = vb.y, b[2] = vb.z, b[3] = vb.w;
+        } else {
+            for (int i = 0; i < 4; ++i)
+                if (n + i < N) a[i] = exc[n + i], b[i] = qexc[n + i];
+        }
+#pragma unroll
+        for (int i = 1; i < 4; ++i) a[i] += a[i - 1], b[i] += b[i - 1];
+        int ia = a[3], ib = b[3];
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1) {
+            const int va = __shfl_up(ia, d), vb = __shfl_up(ib, d);
+            if (lane >= d) ia += va, ib += vb;
+        }
+        if (lane == 63) wsum[0][wave] = ia, wsum[1][wave] = ib;
+        __syncthreads();
+        int oa = ca + ia - a[3], ob = cb + ib - b[3];
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            const int va = wsum[0][i], vb = wsum[1][i];
+            if (i < wave) oa += va, ob += vb;
+            ca += va, cb += vb;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            if (n + i < N) rp[n + i + 1] = oa + a[i], qrp[n + i + 1] = ob + b[i];
+    }
+    if (t == 0) {
+        rp[0] = qrp[0] = 0;
+        out[1] = ca;
+        out[2] = cb;
     }
 }
 
@@ -317,18 +507,56 @@ void launch_codec_to_bf16(const rv12_codec& c, uint16_t* w, hipStream_t st) {
                            c.ev, c.n_exc, c.n, c.k, w);
 }
 
+static void launch_row_windows(const uint16_t* w, int N, int K, int32_t* rbase, int32_t* row_exc, int32_t* cs,
+                               int32_t* part, hipStream_t st) {
+    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(k_row_windows), hipFuncAttributeMaxDynamicSharedMemorySize,
+                              (int)kRowLds);
+    hipLaunchKernelGGL(k_row_windows, dim3((unsigned)min((N + kRowWaves - 1) / kRowWaves, kRowGrid)),
+                       dim3(kRowWaves * 64), kRowLds, st, w, N, K, rbase, row_exc, cs, part);
+}
+
 void launch_pack_plan(const uint16_t* w, int N, int K, int32_t* rbase, int32_t* row_exc, hipStream_t st) {
-    hipLaunchKernelGGL(k_row_base, dim3((unsigned)N), dim3(256), 0, st, w, K, rbase);
-    hipLaunchKernelGGL(k_pack_count, dim3((unsigned)N), dim3(256), 0, st, w, K, rbase, row_exc);
+    launch_row_windows(w, N, K, rbase, row_exc, nullptr, nullptr, st);
+}
+
+static void launch_pack_tiles(const uint16_t* w, int N, int K, const int32_t* rbase, uint32_t* tiles, hipStream_t st) {
+    const int64_t groups = (int64_t)((N + 15) / 16) * (K / 32) * 64;
+    hipLaunchKernelGGL(k_pack_tiles, dim3((unsigned)((groups + 255) / 256)), dim3(256), 0, st, w, N, K, rbase, tiles,
+                       groups);
 }
 
 void launch_pack(const uint16_t* w, int N, int K, const int32_t* rbase, const int32_t* rp, uint32_t* tiles,
                  int32_t* er, int32_t* ec, float* ev, int64_t n_exc, hipStream_t st) {
-    const int64_t groups = (int64_t)((N + 15) / 16) * (K / 32) * 64;
-    hipLaunchKernelGGL(k_pack_tiles, dim3((unsigned)((groups + 255) / 256)), dim3(256), 0, st, w, N, K, rbase, tiles,
-                       groups);
-    if (n_exc > 0)
-        hipLaunchKernelGGL(k_encode_exc, dim3((unsigned)N), dim3(256), 0, st, w, K, 0, rbase, rp, er, ec, ev);
+    launch_pack_tiles(w, N, K, rbase, tiles, st);
+    if (n_exc > 0) launch_exceptions(w, N, K, ExcList{rbase, 0, rp, er, ec, ev}, nullptr, st);
+}
+
+// the histogram and its parts, each row's entries in both lists, row prefix counts
+static size_t padded4(int N) { return ((size_t)N + 3) / 4 * 4; }
+size_t compress_ws_bytes(int N) { return 256 * 8 + ((size_t)kRowGrid * 256 + 2 * padded4(N) + (size_t)N * 256) * 4; }
+
+void launch_compress_plan(const uint16_t* w, int N, int K, int32_t* rbase, int32_t* rp, int32_t* qrp, int32_t* out,
+                          void* ws, hipStream_t st) {
+    int64_t* hist = static_cast<int64_t*>(ws);
+    int32_t* part = reinterpret_cast<int32_t*>(hist + 256);
+    int32_t* exc = part + (size_t)kRowGrid * 256;
+    int32_t* qexc = exc + padded4(N);
+    int32_t* cs = qexc + padded4(N);
+    launch_row_windows(w, N, K, rbase, qexc, cs, part, st);
+    hipLaunchKernelGGL(k_hist_sum, dim3(256 / kHistBins), dim3(256), 0, st, part,
+                       min((N + kRowWaves - 1) / kRowWaves, kRowGrid), hist);
+    hipLaunchKernelGGL(k_row_counts, dim3((unsigned)((N + 255) / 256)), dim3(256), 0, st, hist, cs, N, K, exc, out);
+    hipLaunchKernelGGL(k_row_pointers, dim3(1), dim3(kPlanThreads), 0, st, exc, qexc, N, rp, qrp, out);
+}
+
+void launch_compress_write(const uint16_t* w, int N, int K, int base, const int32_t* rp, int32_t* er, int32_t* ec,
+                           float* ev, int64_t n_exc, const int32_t* rbase, const int32_t* qrp, int32_t* qer,
+                           int32_t* qec, float* qev, int64_t n_qexc, uint32_t* tiles, hipStream_t st) {
+    launch_pack_tiles(w, N, K, rbase, tiles, st);
+    const ExcList a = {nullptr, base, rp, er, ec, ev}, b = {rbase, 0, qrp, qer, qec, qev};
+    if (n_exc > 0 && n_qexc > 0) launch_exceptions(w, N, K, a, &b, st);
+    else if (n_exc > 0) launch_exceptions(w, N, K, a, nullptr, st);
+    else if (n_qexc > 0) launch_exceptions(w, N, K, b, nullptr, st);
 }
 
 void launch_decode(const rv12_matrix& w, int first, int last, void* out, int out_f32, hipStream_t st,
@@ -357,7 +585,7 @@ void launch_encode(const uint16_t* w, int N, int K, int CH, int base, uint8_t* m
 
 void launch_encode_exc(const uint16_t* w, int N, int K, int base, const int32_t* rp, int32_t* er, int32_t* ec,
                        float* ev, hipStream_t st) {
-    hipLaunchKernelGGL(k_encode_exc, dim3((unsigned)N), dim3(256), 0, st, w, K, base, nullptr, rp, er, ec, ev);
+    launch_exceptions(w, N, K, ExcList{nullptr, base, rp, er, ec, ev}, nullptr, st);
 }
 
 }  // namespace rv12

@@ -202,6 +202,12 @@ void launch_pack(const uint16_t* w, int N, int K, const int32_t* rbase, const in
                  int32_t* er, int32_t* ec, float* ev, int64_t n_exc, hipStream_t st);
 void launch_decode(const rv12_matrix& w, int first, int last, void* out, int out_f32, hipStream_t st, int64_t e0,
                    int64_t e1);
+size_t compress_ws_bytes(int N);
+void launch_compress_plan(const uint16_t* w, int N, int K, int32_t* rbase, int32_t* rp, int32_t* qrp, int32_t* out,
+                          void* ws, hipStream_t st);
+void launch_compress_write(const uint16_t* w, int N, int K, int base, const int32_t* rp, int32_t* er, int32_t* ec,
+                           float* ev, int64_t n_exc, const int32_t* rbase, const int32_t* qrp, int32_t* qer,
+                           int32_t* qec, float* qev, int64_t n_qexc, uint32_t* tiles, hipStream_t st);
 void launch_encode_stats(const uint16_t* w, int64_t count, int32_t* hist, hipStream_t st);
 void launch_encode(const uint16_t* w, int N, int K, int CH, int base, uint8_t* m8, uint8_t* e4, int32_t* row_exc,
                    hipStream_t st);

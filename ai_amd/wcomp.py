@@ -122,6 +122,42 @@ def compress(W, CH=256):
     W = W.contiguous()
     if W.data_ptr() % 16:
         W = W.clone()
+    if CH >= 16 and CH % 16 == 0 and lib().rv12_compress_workspace_bytes(N, K):
+        c = _compress_packed(W, N, K, CH, dev)
+    else:
+        c = _compress_arrays(W, N, K, CH, dev)
+    if home.type != "cuda":
+        for k, v in list(c.items()):
+            if torch.is_tensor(v):
+                c[k] = v.to(home)
+    return c
+
+
+def _compress_packed(W, N, K, CH, dev):
+    """The reference keys and the packed form from one pass for the windows and
+    row pointers, one host read (base and the lists' lengths) and one pass for
+    the tiles and lists."""
+    st = _stream(dev)
+    L = lib()
+    i32 = dict(dtype=torch.int32, device=dev)
+    rp, qrp, rbase, out = torch.empty(N + 1, **i32), torch.empty(N + 1, **i32), torch.empty(N, **i32), torch.empty(3, **i32)
+    ws = torch.empty(L.rv12_compress_workspace_bytes(N, K), dtype=torch.uint8, device=dev)
+    tiles = torch.empty(L.rv12_tiles_bytes(N, K) // 4, **i32)
+    check(L.rv12_compress_plan(_ptr(W), N, K, _ptr(rbase), _ptr(rp), _ptr(qrp), _ptr(out), _ptr(ws), ws.numel(), st),
+          "compress")
+    base, E, Q = out.tolist()
+    del ws
+    er, ec, qer, qec = (torch.empty(n, **i32) for n in (E, E, Q, Q))
+    ev, qev = (torch.empty(n, dtype=torch.float32, device=dev) for n in (E, Q))
+    check(L.rv12_compress_write(_ptr(W), N, K, base, _ptr(rp), E, _ptr(er), _ptr(ec), _ptr(ev), _ptr(rbase), _ptr(qrp),
+                                Q, _ptr(tiles), tiles.numel() * 4, _ptr(qer), _ptr(qec), _ptr(qev), st), "compress")
+    return Codec12(base=base, rp=rp, er=er, ec=ec, ev=ev, N=N, K=K, CH=CH, q16_tiles=tiles, q16_rbase=rbase,
+                   q16_rp=qrp, q16_er=qer, q16_ec=qec, q16_ev=qev)
+
+
+def _compress_arrays(W, N, K, CH, dev):
+    """compress() of a matrix without a packed form (K or CH off its steps), whose
+    dict keeps m8 and e4."""
     st = _stream(dev)
     L = lib()
     hist = torch.empty(256, dtype=torch.int32, device=dev)
@@ -140,15 +176,10 @@ def compress(W, CH=256):
     if E:
         check(L.rv12_encode_exc(_ptr(W), N, K, base, _ptr(rp), _ptr(er), _ptr(ec), _ptr(ev), st), "compress")
     c = Codec12(base=base, rp=rp, er=er, ec=ec, ev=ev, N=N, K=K, CH=CH)
-    if K % 32 == 0 and CH % 16 == 0:
+    if CH > 0 and K % 32 == 0 and CH % 16 == 0:
         c.update(pack(W))
-        del m8, e4
     else:  # no packed form for this K: the dict keeps the reference arrays
         c["m8"], c["e4"] = m8, e4
-    if home.type != "cuda":
-        for k, v in list(c.items()):
-            if torch.is_tensor(v):
-                c[k] = v.to(home)
     return c
 
 

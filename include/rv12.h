@@ -125,6 +125,23 @@ int rv12_pack_plan(const uint16_t* w, int n, int k, int32_t* rbase, int32_t* row
 int rv12_pack(const uint16_t* w, int n, int k, const int32_t* rbase, const int32_t* rp, int64_t n_exc,
               uint32_t* tiles, size_t tiles_bytes, int32_t* er, int32_t* ec, float* ev, void* stream);
 
+/* Both forms of one matrix at once, as compress() keeps them (the reference
+ * codec's base, row pointers and exception list, wcomp.py:13-32, without m8 / e4;
+ * the packed form), in two calls with one host step between them:
+ *   rv12_compress_plan   rbase[n] and qrp[n + 1] of the packed form, rp[n + 1] of
+ *                        the codec, out[3] = {base, rp[n], qrp[n]} (int32, device);
+ *                        ws: rv12_compress_workspace_bytes(n, k) bytes, 16-byte
+ *                        aligned (0 for shapes the calls reject)
+ *   (host: read out, allocate the lists)
+ *   rv12_compress_write  tiles and both lists: what rv12_encode_exc and rv12_pack
+ *                        write */
+size_t rv12_compress_workspace_bytes(int n, int k);
+int rv12_compress_plan(const uint16_t* w, int n, int k, int32_t* rbase, int32_t* rp, int32_t* qrp, int32_t* out,
+                       void* ws, size_t ws_bytes, void* stream);
+int rv12_compress_write(const uint16_t* w, int n, int k, int base, const int32_t* rp, int64_t n_exc, int32_t* er,
+                        int32_t* ec, float* ev, const int32_t* rbase, const int32_t* qrp, int64_t n_qexc,
+                        uint32_t* tiles, size_t tiles_bytes, int32_t* qer, int32_t* qec, float* qev, void* stream);
+
 /* The bf16 matrix w[n, k] a codec dict encodes (the inverse of compress(),
  * bit for bit; the reference's decompress, wcomp.py:35-45, ends with a
  * .bfloat16() that would also map every NaN payload to one NaN).  Used to

@@ -178,3 +178,32 @@ def test_random_draws_against_the_oracle_codec():
         assert np.array_equal(c["ev"].cpu().numpy().view(np.uint32), np.asarray(ref["ev"]).view(np.uint32)), d
         back = wcomp.decompress(c).view(torch.int16).cpu().numpy().view(np.uint16)
         assert np.array_equal(back, bits), d
+
+
+@pytest.mark.parametrize("N,K,every", [(1, 32, 1), (3, 2080, 7), (17, 512, 0), (2050, 96, 5), (4097, 64, 1), (9000, 32, 40)])
+def test_compress_in_one_pass_matches_the_separate_calls(N, K, every):
+    """base, row pointers, both exception lists, windows and tiles of compress()
+    equal those of rv12_encode* and rv12_pack* called one after the other and
+    the oracle's: rows past one wave's stride and one tile of the plan's scan,
+    K off the 512- and 2048-weight chunks, no exception, one in `every` weights
+    or nothing else."""
+    from ai_amd import wcomp
+    from oracle import codec
+    rng = np.random.default_rng(N + K)
+    w = (rng.standard_normal((N, K)) * 0.02).astype(np.float32)
+    w = np.copysign(np.clip(np.abs(w), 2.0 ** -10, 0.12), w)
+    if every:
+        w.reshape(-1)[::every] = rng.choice([3e4, 1e-30, 0.0, -1e-39, np.inf], w.reshape(-1)[::every].size)
+    bits = codec.f32_to_bf16_rne(w)
+    W = _w(bits)
+    c, d = wcomp.compress(W, CH=32), wcomp._compress_arrays(W, N, K, 32, W.device)
+    assert list(c) == list(d) and c["base"] == d["base"]
+    for k in list(c):
+        if torch.is_tensor(c[k]):
+            assert c[k].dtype == d[k].dtype and c[k].shape == d[k].shape, k
+            assert torch.equal(c[k].view(torch.int32), d[k].view(torch.int32)), k
+    o = codec.compress(bits, CH=32)
+    assert c["base"] == o["base"]
+    for k in ("rp", "er", "ec"):
+        assert np.array_equal(c[k].cpu().numpy(), o[k]), k
+    assert np.array_equal(c["ev"].cpu().numpy().view(np.uint32), np.asarray(o["ev"]).view(np.uint32))
