@@ -28,7 +28,8 @@ EXPORTS = ("rv12_abi_version", "rv12_strerror", "rv12_tiles_bytes", "rv12_pack_p
            "rv12_attn_batch_workspace_bytes", "rv12_rope_attn_batch", "rv12_prefill_attn_workspace_bytes",
            "rv12_prefill_rope_attn", "rv12_prefill_workspace_bytes",
            "rv12_prefill_linear", "rv12_decode_advance",
-           "rv12_compress_workspace_bytes", "rv12_compress_plan", "rv12_compress_write")
+           "rv12_compress_workspace_bytes", "rv12_compress_plan", "rv12_compress_write",
+           "rv12_prefill_parts_workspace_bytes", "rv12_prefill_linear_parts")
 ABI_VERSION = 8
 STATIC_SCRATCH_BYTES = 8 << 20  # RV12_STATIC_SCRATCH_BYTES
 
@@ -130,6 +131,10 @@ def lib():
         L.rv12_prefill_workspace_bytes.argtypes = [I, I, I]
         L.rv12_prefill_linear.restype = I
         L.rv12_prefill_linear.argtypes = [ctypes.POINTER(Matrix), P, P, I, P, F, I, P, SZ, P]
+        L.rv12_prefill_parts_workspace_bytes.restype = SZ
+        L.rv12_prefill_parts_workspace_bytes.argtypes = [I, I, I, I]
+        L.rv12_prefill_linear_parts.restype = I
+        L.rv12_prefill_linear_parts.argtypes = [ctypes.POINTER(Matrix), P, P, I, P, F, I, I, P, SZ, P]
         L.rv12_decode_advance.restype = I
         L.rv12_decode_advance.argtypes = [P, P, ctypes.c_int64, I, P, P, ctypes.c_int64, P, P, P, P]
         L.rv12_attn_batch_workspace_bytes.restype = SZ

@@ -578,23 +578,34 @@ int rv12_head_argmax(const rv12_matrix* w, const float* x, int t, const uint16_t
 
 size_t rv12_prefill_workspace_bytes(int n, int k, int t) {
     if (n < 1 || k < 32 || k % 32 || k > kMaxK || t < 1 || t > kMaxPrefillTokens) return 0;
-    return prefill_ws_bytes(n, k, t);
+    return prefill_ws_bytes(n, k, t, 2);
+}
+
+size_t rv12_prefill_parts_workspace_bytes(int n, int k, int t, int parts) {
+    if (n < 1 || k < 32 || k % 32 || k > kMaxK || t < 1 || t > kMaxPrefillTokens || parts < 2 || parts > 3) return 0;
+    return prefill_ws_bytes(n, k, t, parts);
 }
 
 int rv12_prefill_linear(const rv12_matrix* w, const float* x, float* y, int t, const uint16_t* lnw, float eps,
                         int mode, void* ws, size_t ws_bytes, void* stream) {
+    return rv12_prefill_linear_parts(w, x, y, t, lnw, eps, mode, 2, ws, ws_bytes, stream);
+}
+
+int rv12_prefill_linear_parts(const rv12_matrix* w, const float* x, float* y, int t, const uint16_t* lnw, float eps,
+                              int mode, int parts, void* ws, size_t ws_bytes, void* stream) {
     int rc = check_matrix(w);
     if (rc) return rc;
     if (!x || !y) return RV12_E_NULL;
     if (mode < 0 || mode > 2) return RV12_E_MODE;
+    if (parts < 2 || parts > 3) return RV12_E_CONFIG;
     if (lnw && mode == 2) return RV12_E_MODE;  // the RMS prologue belongs to the plain linear
     if (lnw && (uintptr_t)lnw % 16) return RV12_E_ALIGN;
     if (t < 1 || t > kMaxPrefillTokens) return RV12_E_TOKENS;
     if (!aligned16(x) || !aligned16(y)) return RV12_E_ALIGN;
-    const size_t need = prefill_ws_bytes(w->n, w->k, t);
+    const size_t need = prefill_ws_bytes(w->n, w->k, t, parts);
     if (!ws || ws_bytes < need) return RV12_E_WORKSPACE;
     if (!aligned16(ws)) return RV12_E_ALIGN;
-    launch_prefill(*w, x, y, t, mode, lnw, eps, ws, (hipStream_t)stream);
+    launch_prefill(*w, x, y, t, mode, lnw, eps, parts, ws, (hipStream_t)stream);
     return launch_status();
 }
 

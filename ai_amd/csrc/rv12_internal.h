@@ -189,13 +189,13 @@ void launch_pick(const float* v, const int32_t* ix, int64_t n, int64_t stride, i
                  int64_t* ids, hipStream_t st);
 // --- prefill linear (k_prefill_x + k_prefill_mm), any T
 constexpr int kMaxPrefillTokens = 1 << 16;
-size_t prefill_ws_bytes(int N, int K, int T);
-int prefill_splits(int N, int K, int T);
+size_t prefill_ws_bytes(int N, int K, int T, int parts);
+int prefill_splits(int N, int K, int T, int parts);
 void launch_decode_advance(const int64_t* ids, const uint16_t* emb, int64_t vocab, int hidden, float* x,
                            int64_t* out, int64_t out_len, int64_t* steps, int64_t* pos, int64_t* tok,
                            hipStream_t st);
 void launch_prefill(const rv12_matrix& w, const float* x, float* y, int T, int mode, const uint16_t* lnw, float eps,
-                    void* ws, hipStream_t st);
+                    int parts, void* ws, hipStream_t st);
 void launch_codec_to_bf16(const rv12_codec& c, uint16_t* w, hipStream_t st);
 void launch_pack_plan(const uint16_t* w, int N, int K, int32_t* rbase, int32_t* row_exc, hipStream_t st);
 void launch_pack(const uint16_t* w, int N, int K, const int32_t* rbase, const int32_t* rp, uint32_t* tiles,

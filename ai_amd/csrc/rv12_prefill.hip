@@ -22,7 +22,12 @@
 //      out closer to 64 bits than before (24576 x 4096 over 2048 tokens:
 //      relative error 7.0e-7 -> 2.3e-7; 1024 x 3072 over 301: 1.95e-7 ->
 //      1.79e-7).  A tile with a token whose values the float16 parts would not
-//      hold (see tok_exp) keeps the three bf16 parts.
+//      hold (see tok_exp) keeps the three bf16 parts, and so does a call that
+//      asks for them (parts = 3): the prompt's qkv, whose keys and values are
+//      rounded into the cache and must stay, bit for bit, what earlier prompts
+//      left there (with two parts one in 10^4 bf16 entries falls on the other
+//      side of its rounding; the three parts cost the Qwen3-8B layer over 2048
+//      tokens about 40 us of 2036).
 //      Workgroup = 256 rows x 128 tokens, 8 waves of 64 rows x 64 tokens.  Per
 //      32-column step the workgroup's 16 row blocks' Q16 tiles and the B parts
 //      go from memory straight into a ring of LDS slots (buffer loads with the
@@ -85,13 +90,12 @@ constexpr int kPfRing3 = 4;
 constexpr int kPfSlot3 = kPfSlotA + kPfTokBlocks * 3 * 64;
 static_assert((size_t)kPfRing3 * kPfSlot3 * 16 <= kPfLds, "LDS of one workgroup");
 constexpr int kPfOps3 = kPfAPerWave + kPfTokBlocks * 3 / kPfWaves;
-constexpr int kPfWait3 = kPfOps3 * (kPfRing3 - 1);  // the loads issued after step s's
+constexpr int kPfWait3 = kPfOps3 * (kPfRing3 - 2);  // the loads issued after step s + 1's, at the top of step s
 static_assert(kPfWait3 < 64 && kPfWait2 < 64, "vmcnt holds 6 bits");
 // s_waitcnt immediates (gfx9 encoding): vmcnt(n) and lgkmcnt(0), expcnt not
 // waited for; vmcnt(n) alone
 constexpr int waitcnt_vm_lgkm0(int n) { return (n & 15) | ((n >> 4) << 14) | (7 << 4); }
 constexpr int waitcnt_vm(int n) { return waitcnt_vm_lgkm0(n) | (15 << 8); }
-constexpr int waitcnt_lgkm0() { return waitcnt_vm_lgkm0(63); }
 
 // 12 or 16 bytes per lane from a descriptor straight into LDS (lane l at
 // d + 16 bytes l)
@@ -215,14 +219,14 @@ constexpr int kPpThreads = 256;
 __global__ __launch_bounds__(kPpThreads) void k_prefill_parts(const float* __restrict__ x, int T, int K, int xs,
                                                               int m2, const uint16_t* __restrict__ lnw,
                                                               const int* __restrict__ E, u32x4* __restrict__ xb,
-                                                              float* __restrict__ xt, int tp) {
+                                                              float* __restrict__ xt, int tp, int parts) {
     const int tok = threadIdx.x & 31, k8 = threadIdx.x >> 5;
     const int t = blockIdx.x * 32 + tok;
     const int kc = blockIdx.y * 64 + k8 * 8;
     const int nsteps = K >> 5;
     float v[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
     if (t < T && kc < K) prefill_xprime(x + (int64_t)t * xs, K, kc, m2 != 0, lnw, v);
-    const bool wide = __ballot(wide_lanes(E, (int)(blockIdx.x * 32) / kPfTokens * kPfTokens, T) & 1) != 0;
+    const bool wide = parts == 3 || __ballot(wide_lanes(E, (int)(blockIdx.x * 32) / kPfTokens * kPfTokens, T) & 1) != 0;
     if (kc >= K) return;
     float* xc = xt + (int64_t)kc * tp + t;
 #pragma unroll
@@ -281,7 +285,8 @@ __global__ __launch_bounds__(kPfThreads) void k_prefill_mm(const uint32_t* __res
                                                            const int32_t* __restrict__ ec,
                                                            const float* __restrict__ ev, const float* __restrict__ xt,
                                                            int tp, const float* __restrict__ R, float* __restrict__ y,
-                                                           float* __restrict__ part, int N, int K, int T, int add) {
+                                                           float* __restrict__ part, int N, int K, int T, int add,
+                                                           int parts) {
     extern __shared__ u32x4 bs[];  // the ring's slots: A tiles and B parts of consecutive steps
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -346,11 +351,13 @@ __global__ __launch_bounds__(kPfThreads) void k_prefill_mm(const uint32_t* __res
     };
     // steps 0 .. kPfRing2 - 2 into slots 0 .. (a wide tile starts over: what these
     // loads bring is in bounds and unused)
+    if (parts == 2) {
 #pragma unroll
-    for (int j = 0; j < kPfRing2 - 1; ++j)
+        for (int j = 0; j < kPfRing2 - 1; ++j)
 #pragma unroll
-        for (int i = 0; i < kPfOps2; ++i) load_op(i, j * kPfSlot2, j);
-    const bool wide = __ballot(wl & 1) != 0;
+            for (int i = 0; i < kPfOps2; ++i) load_op(i, j * kPfSlot2, j);
+    }
+    const bool wide = parts == 3 || __ballot(wl & 1) != 0;
 
     if (!wide) {
         const int ra0 = wr * kPfWB * 64 + lane, rb0 = kPfSlotA + wc * kPfWT * 128 + lane;
@@ -454,41 +461,58 @@ __global__ __launch_bounds__(kPfThreads) void k_prefill_mm(const uint32_t* __res
             for (int j = 0; j < 3; ++j)
                 load_lds16(rb, d + kPfSlotA + wave * 64 + j * kPfThreads, boff3[j], sb);
         };
-        // steps 0 .. 3 into slots 0 .. 3, then per step: its loads landed,
-        // barrier, its fragments and 48 MFMAs, barrier, the step 4 ahead
-        // into its slot.
-#pragma unroll
-        for (int i = 0; i < kPfRing3; ++i) load_step(i, i);
-        int slot = 0;
-        for (int s = 0; s < s_hi - s_lo; ++s) {
-            asm volatile("" ::: "memory");
-            __builtin_amdgcn_s_waitcnt(waitcnt_vm(kPfWait3));
-            __builtin_amdgcn_s_barrier();
-            asm volatile("" ::: "memory");
+        // this wave's fragments of the step in slot `slot`: its 4 row blocks' A
+        // groups and 3 parts x 4 token blocks of B, part-major so the first
+        // part's MFMAs wait only for its own reads
+        auto read_frags = [&](u32x3 (&fa)[kPfWB], u32x4 (&fb)[3][kPfWT], int slot) {
             const u32x4* d = bs + slot * kPfSlot3;
-            u32x4 a[kPfWB];
 #pragma unroll
-            for (int b = 0; b < kPfWB; ++b) {
-                const u32x3 r = *reinterpret_cast<const u32x3*>(d + (wr * kPfWB + b) * 64 + lane);
-                uint32_t pr[4];
-                unpack_pairs(r.x, r.y, r.z, pr);
-                a[b] = u32x4{pr[0], pr[1], pr[2], pr[3]};
-            }
+            for (int b = 0; b < kPfWB; ++b) fa[b] = *reinterpret_cast<const u32x3*>(d + (wr * kPfWB + b) * 64 + lane);
             const u32x4* src = d + kPfSlotA + wc * kPfWT * 192 + lane;
 #pragma unroll
             for (int q = 0; q < 3; ++q)
 #pragma unroll
-                for (int c = 0; c < kPfWT; ++c) {
-                    const u32x4 bf = src[c * 192 + q * 64];
+                for (int c = 0; c < kPfWT; ++c) fb[q][c] = src[c * 192 + q * 64];
+        };
+        // steps 0-3 into slots 0-3, all landed; step 0's fragments read
 #pragma unroll
-                    for (int b = 0; b < kPfWB; ++b) acc[b][c] = mfma(a[b], bf, acc[b][c]);
+        for (int i = 0; i < kPfRing3; ++i) load_step(i, i);
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        u32x3 fa[2][kPfWB];
+        u32x4 fb[2][3][kPfWT];
+        read_frags(fa[0], fb[0], 0);
+        // Step s: wait for this wave's loads of step s + 1 and its fragment reads
+        // of step s; barrier; step s + 4 into slot s % 4; the fragments of step
+        // s + 1 read while the 48 MFMAs of step s run.  Whole rounds of the
+        // unroll: steps past the split read zeros and add nothing.
+        for (int s0 = 0; s0 < s_hi - s_lo; s0 += kPfRing3) {
+#pragma unroll
+            for (int u = 0; u < kPfRing3; ++u) {
+                asm volatile("" ::: "memory");
+                __builtin_amdgcn_s_waitcnt(waitcnt_vm_lgkm0(kPfWait3));
+                __builtin_amdgcn_s_barrier();
+                asm volatile("" ::: "memory");
+                load_step(u, s0 + u + kPfRing3);
+                read_frags(fa[(u + 1) & 1], fb[(u + 1) & 1], (u + 1) % kPfRing3);
+                asm volatile("" ::: "memory");
+                __builtin_amdgcn_sched_barrier(0);
+                u32x4 a[kPfWB];
+#pragma unroll
+                for (int b = 0; b < kPfWB; ++b) {
+                    uint32_t pr[4];
+                    unpack_pairs(fa[u & 1][b].x, fa[u & 1][b].y, fa[u & 1][b].z, pr);
+                    a[b] = u32x4{pr[0], pr[1], pr[2], pr[3]};
                 }
-            asm volatile("" ::: "memory");
-            __builtin_amdgcn_s_waitcnt(waitcnt_lgkm0());
-            __builtin_amdgcn_s_barrier();
-            asm volatile("" ::: "memory");
-            load_step(slot, s + kPfRing3);
-            slot = slot + 1 == kPfRing3 ? 0 : slot + 1;
+#pragma unroll
+                for (int q = 0; q < 3; ++q)
+#pragma unroll
+                    for (int b = 0; b < kPfWB; ++b)
+#pragma unroll
+                        for (int c = 0; c < kPfWT; ++c) acc[b][c] = mfma(a[b], fb[u & 1][q][c], acc[b][c]);
+            }
         }
     }
     // the last loads (zeros into slots nobody reads) land before the
@@ -674,7 +698,9 @@ __global__ __launch_bounds__(256) void k_prefill_reduce(const float* __restrict_
 // reduce pass costs 4 us + (S + 1) T N floats at 5 TB/s (1024 x 3072 over 301
 // tokens: 92 us unsplit, 36 with 12 splits; 4096 x 4096 over 2048, one full
 // round: 160 unsplit, 183 with 2).  No split below 8 steps.
-int prefill_splits(int N, int K, int T) {
+// Three parts: a step 1.4 us and 10 us a round, 3 us + the floats for the reduce
+// pass, the splits this path has always had, so that its sums keep their order.
+int prefill_splits(int N, int K, int T, int parts) {
     const int64_t nx = ((int64_t)N + 16 * kPfRowBlocks - 1) / (16 * kPfRowBlocks);
     const int tp = prefill_tokens_padded(T), nsteps = K / 32;
     const int64_t G = nx * (tp / kPfTokens);
@@ -682,11 +708,17 @@ int prefill_splits(int N, int K, int T) {
     double best_us = 0.0;
     for (int S = 1; S <= 16; ++S) {
         if (S > 1 && nsteps / S < 8) break;
-        const double steps = (nsteps + S - 1) / S;
-        const double last = (double)(G * S % 256) / 256;
-        double us = (double)(G * S / 256) * (steps * 1.0 + 8.0);
-        if (last > 0) us += steps * (0.8 + 0.2 * last * last) + 8.0;
-        if (S > 1) us += 4.0 + (double)(S + 1) * tp * N * 4 / 5e6;
+        double us;
+        if (parts == 3) {
+            us = (double)((G * S + 255) / 256) * ((double)nsteps / S * 1.4 + 10.0);
+            if (S > 1) us += 3.0 + (double)(S + 1) * tp * N * 4 / 5e6;
+        } else {
+            const double steps = (nsteps + S - 1) / S;
+            const double last = (double)(G * S % 256) / 256;
+            us = (double)(G * S / 256) * (steps * 1.0 + 8.0);
+            if (last > 0) us += steps * (0.8 + 0.2 * last * last) + 8.0;
+            if (S > 1) us += 4.0 + (double)(S + 1) * tp * N * 4 / 5e6;
+        }
         if (S == 1 || us < best_us) {
             best = S;
             best_us = us;
@@ -695,15 +727,15 @@ int prefill_splits(int N, int K, int T) {
     return best;
 }
 
-size_t prefill_ws_bytes(int N, int K, int T) {
+size_t prefill_ws_bytes(int N, int K, int T, int parts) {
     const size_t tp = (size_t)prefill_tokens_padded(T);
-    const int S = prefill_splits(N, K, T);
+    const int S = prefill_splits(N, K, T, parts);
     // parts (room for three), E and R, transposed x', split partials
     return tp * (size_t)K * 10 + tp * 8 + (S > 1 ? (size_t)S * tp * (size_t)N * 4 : 0);
 }
 
 void launch_prefill(const rv12_matrix& w, const float* x, float* y, int T, int mode, const uint16_t* lnw, float eps,
-                    void* ws, hipStream_t st) {
+                    int parts, void* ws, hipStream_t st) {
     const int K = w.k, N = w.n;
     const int tp = prefill_tokens_padded(T);
     u32x4* xb = reinterpret_cast<u32x4*>(ws);
@@ -713,18 +745,18 @@ void launch_prefill(const rv12_matrix& w, const float* x, float* y, int T, int m
     float* part = xt + (size_t)tp * K;
     const int xs = mode == 2 ? 2 * K : K;
     const int m2 = mode == 2 ? 1 : 0;
-    const int S = prefill_splits(N, K, T);
+    const int S = prefill_splits(N, K, T, parts);
     hipLaunchKernelGGL(k_prefill_stats, dim3(tp / (kPsThreads / 64)), dim3(kPsThreads), 0, st, x, T, K, xs, m2, lnw, eps,
                        E, R);
     hipLaunchKernelGGL(k_prefill_parts, dim3(tp / 32, (K + 63) / 64), dim3(kPpThreads), 0, st, x, T, K, xs, m2, lnw, E,
-                       xb, xt, tp);
+                       xb, xt, tp, parts);
     const int64_t nblk = ((int64_t)N + 15) / 16;
     const dim3 grid((unsigned)((nblk + kPfRowBlocks - 1) / kPfRowBlocks * (tp / kPfTokens)), (unsigned)S);
     const auto kern = lnw ? k_prefill_mm<true> : k_prefill_mm<false>;
     (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
                               (int)kPfLds);
     hipLaunchKernelGGL(kern, grid, dim3(kPfThreads), kPfLds, st, reinterpret_cast<const uint32_t*>(w.tiles), w.rbase, xb,
-                       E, w.rp, w.er, w.ec, w.ev, xt, tp, R, y, part, N, K, T, mode != 0 ? 1 : 0);
+                       E, w.rp, w.er, w.ec, w.ev, xt, tp, R, y, part, N, K, T, mode != 0 ? 1 : 0, parts);
     if (S > 1) {
         const int V = N % 4 == 0 ? 4 : 1;
         const dim3 rgrid((unsigned)((N + 256 * V - 1) / (256 * V)), (unsigned)min(T, 65535));

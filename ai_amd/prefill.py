@@ -50,9 +50,10 @@ def enabled(n=None):
 _WS = {}  # device -> workspace of the prefill linear (the split activations)
 
 
-def _linear(x, c, y, mode, lnw=None, eps=1e-6):
+def _linear(x, c, y, mode, lnw=None, eps=1e-6, parts=2):
     """y (=|+=) W x' over every token row of x (fp32 [T, K], [T, 2K] in mode
-    2); lnw (bf16 [K]) fuses the row's RMSNorm, as gemvc1 does."""
+    2); lnw (bf16 [K]) fuses the row's RMSNorm, as gemvc1 does.  parts: the
+    16-bit parts of each activation, 2 or 3."""
     import ctypes
     from . import _lib
     T = x.shape[0]
@@ -64,16 +65,16 @@ def _linear(x, c, y, mode, lnw=None, eps=1e-6):
     if lnw is not None and (lnw.dtype != torch.bfloat16 or not lnw.is_contiguous() or lnw.numel() < K):
         raise ValueError("prefill: lnw must be a contiguous bf16 vector of K entries")
     L = _lib.lib()
-    need = L.rv12_prefill_workspace_bytes(N, K, T)
+    need = L.rv12_prefill_parts_workspace_bytes(N, K, T, parts)
     if need == 0:
         raise ValueError("prefill: too many tokens")
     key = str(x.device)
     if key not in _WS or _WS[key].numel() < need:
         _WS[key] = torch.empty(need, dtype=torch.uint8, device=x.device)
     ws = _WS[key]
-    rc = L.rv12_prefill_linear(ctypes.byref(wcomp._matrix(c)), ctypes.c_void_p(x.data_ptr()),
+    rc = L.rv12_prefill_linear_parts(ctypes.byref(wcomp._matrix(c)), ctypes.c_void_p(x.data_ptr()),
                                ctypes.c_void_p(y.data_ptr()), T,
-                               None if lnw is None else ctypes.c_void_p(lnw.data_ptr()), float(eps), int(mode),
+                               None if lnw is None else ctypes.c_void_p(lnw.data_ptr()), float(eps), int(mode), parts,
                                ctypes.c_void_p(ws.data_ptr()), ws.numel(),
                                ctypes.c_void_p(torch.cuda.current_stream(x.device).cuda_stream))
     _lib.check(rc, "prefill")
@@ -122,7 +123,9 @@ def layer(eng, l, weights, x, start, kc, vc, gguf=False):
     s = eng.small[l]
     bf = lambda t: t.to(torch.bfloat16).contiguous()
     qkv = torch.empty(T, (H + 2 * KV) * HD, device=x.device)
-    matrix(x, W["qkv"], qkv, lnw=bf(s["ln1"]), eps=eps)
+    # three parts: the keys and values rounded into the cache stay bit for bit
+    # what earlier prompts left there
+    _linear(x, W["qkv"], qkv, 0, bf(s["ln1"]), eps, parts=3)
     f32 = lambda t: t.float().contiguous()
     att = torch.empty(T, H * HD, device=x.device)
     _attn(eng, kc).prefill(qkv, f32(s["qn"]), f32(s["kn"]), f32(eng.inv), _pos(x.device, start), kc, vc, att, T)

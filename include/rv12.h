@@ -264,6 +264,12 @@ int rv12_gemm_static(const rv12_matrix* w, const float* x, float* y, int t, cons
 size_t rv12_prefill_workspace_bytes(int n, int k, int t);
 int rv12_prefill_linear(const rv12_matrix* w, const float* x, float* y, int t, const uint16_t* lnw, float eps,
                         int mode, void* ws, size_t ws_bytes, void* stream);
+/* The same with the parts per activation given: 2 (as rv12_prefill_linear) or 3,
+ * bf16 always, each sum in the order it has always had (for outputs that are
+ * rounded and kept, the prompt's keys and values). */
+size_t rv12_prefill_parts_workspace_bytes(int n, int k, int t, int parts);
+int rv12_prefill_linear_parts(const rv12_matrix* w, const float* x, float* y, int t, const uint16_t* lnw, float eps,
+                              int mode, int parts, void* ws, size_t ws_bytes, void* stream);
 
 /* Bit-exact decode of rows [first, last) to bf16 bits (out_f32 == 0, out is
  * uint16[last-first, K]) or to float32 (out_f32 != 0, out is float[last-first, K]).

@@ -270,3 +270,26 @@ def test_tokens_over_many_exponents(N, T, big):
     want, mag = x.astype(np.float64) @ w64.T, np.abs(x.astype(np.float64)) @ np.abs(w64).T
     err = np.abs(y.cpu().numpy() - want)
     assert np.all(err <= 4 * (K + 8) * 2.0 ** -24 * mag + 1e-30), float((err / mag).max())
+
+
+@pytest.mark.parametrize("T,K", [(17, 160), (300, 512), (130, 1056)])
+def test_three_parts_on_request(T, K):
+    """parts = 3: the linear whose outputs are rounded into the caches; steps off
+    the four-slot ring, split and unsplit, the RMS prologue."""
+    from ai_amd import prefill, wcomp
+    rng = np.random.default_rng(T)
+    N = 301
+    bits = codec.f32_to_bf16_rne((rng.standard_normal((N, K)) * 0.02).astype(np.float32))
+    c = wcomp.compress(torch.from_numpy(bits.view(np.int16)).view(torch.bfloat16).cuda(), CH=32)
+    x = rng.standard_normal((T, K)).astype(np.float32)
+    lw = codec.f32_to_bf16_rne((1 + 0.1 * rng.standard_normal(K)).astype(np.float32))
+    y = torch.zeros(T, N, device="cuda")
+    prefill._linear(torch.from_numpy(x).cuda(), c, y, 0, torch.from_numpy(lw.view(np.int16)).view(torch.bfloat16).cuda(),
+                    1e-6, parts=3)
+    x64 = x.astype(np.float64)
+    x64 = x64 / np.sqrt((x64 ** 2).mean(1, keepdims=True) + 1e-6) * codec.bf16_to_f32(lw).astype(np.float64)
+    w64 = codec.bf16_to_f32(bits).astype(np.float64)
+    err, mag = np.abs(y.cpu().numpy() - x64 @ w64.T), np.abs(x64) @ np.abs(w64).T
+    assert np.all(err <= 4 * (K + 8) * 2.0 ** -24 * mag), float((err / mag).max())
+    with pytest.raises(ValueError):
+        prefill._linear(torch.from_numpy(x).cuda(), c, y, 0, parts=4)
