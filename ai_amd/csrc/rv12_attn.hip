@@ -532,8 +532,9 @@ typedef short s16x4 __attribute__((ext_vector_type(4)));  // four bf16 MFMA oper
 // (it has the most positions); with S > 1 splits (the batched pass: T <= 16,
 // one tile) split sp covers blocks [sp nkb / S, (sp + 1) nkb / S) of the
 // tile's nkb blocks of 16 positions and writes (sums, m, l) partials for
-// k_attn_combine; workgroup = the G query heads of kv head g, one wave per head,
-// all reading the same cache rows.  Per block of 16 positions a wave computes
+// k_attn_combine; workgroup = the G query heads of kv head g, PW waves per head
+// (1 with S > 1), all reading the same cache rows; wave part w of a head takes
+// the blocks w, w + PW, .. and the parts' (sums, m, l) join in LDS at the end.  Per block of 16 positions a wave computes
 // the scores transposed, S^T = K . Q^T (rows = positions, columns = its 16
 // tokens), so each lane holds 4 positions of one token: the online softmax
 // (running max m, rescale exp(m_old - m_new), running sum) needs two lane
@@ -559,7 +560,9 @@ __global__ __launch_bounds__(512) void k_prefill_attn(AttnParams p) {
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     const int q4 = lane >> 4, c16 = lane & 15;
     const int H = p.n_heads, KV = p.n_kv, G = H / KV;
-    const int g = blockIdx.y, h = g * G + wv;
+    const int PW = (int)(blockDim.x >> 6) / G;  // waves per head (S = 1), wave wv: head wv % G, part wv / G
+    const int hd = wv % G, part = wv / G;
+    const int g = blockIdx.y, h = g * G + hd;
     const int S = gridDim.z, sp = blockIdx.z;  // position splits (S > 1: T <= 16, one token tile)
     const int T = p.T;
     const int ntile = (T + 15) >> 4;
@@ -569,9 +572,9 @@ __global__ __launch_bounds__(512) void k_prefill_attn(AttnParams p) {
     float* orow = p.out + (int64_t)min(tq, T - 1) * H * HD + h * HD;
     // split partials [n_kv][S][R][HD + 2], row tq G + (h - g G) of R = T G
     float* prow =
-        S > 1 ? p.part + (((int64_t)g * S + sp) * T * G + (int64_t)min(tq, T - 1) * G + wv) * (HD + 2) : nullptr;
+        S > 1 ? p.part + (((int64_t)g * S + sp) * T * G + (int64_t)min(tq, T - 1) * G + hd) * (HD + 2) : nullptr;
     if (p0 < 0 || p0 + T > p.maxt) {  // a block outside the cache: zeros, as the prologue writes nothing
-        if (tq < T && q4 == 0) {
+        if (tq < T && q4 == 0 && part == 0) {
             if (S == 1) {
                 for (int d = 0; d < HD; ++d) orow[d] = 0.0f;
             } else {  // partials that combine to zeros: acc 0, and l = 1 on split 0 only
@@ -656,8 +659,8 @@ __global__ __launch_bounds__(512) void k_prefill_attn(AttnParams p) {
     for (int d = 0; d < DT; ++d) o[d] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
     float m = -INFINITY, l = 0.0f;
     const int qpos = (int)p0 + tq;  // the last position this lane's token sees
-    if (kb0 < kb1) load_block(kb0);
-    for (int kb = kb0; kb < kb1; ++kb) {
+    if (kb0 + part < kb1) load_block(kb0 + part);
+    for (int kb = kb0 + part; kb < kb1; kb += PW) {
         uint32_t kcur[NA][KWD], vcur[4][VWD];
 #pragma unroll
         for (int a = 0; a < NA; ++a)
@@ -667,7 +670,7 @@ __global__ __launch_bounds__(512) void k_prefill_attn(AttnParams p) {
         for (int j = 0; j < 4; ++j)
 #pragma unroll
             for (int i = 0; i < VWD; ++i) vcur[j][i] = vw[j][i];
-        if (kb + 1 < kb1) load_block(kb + 1);
+        if (kb + PW < kb1) load_block(kb + PW);
         // scores of positions kb 16 + 4 q4 + r for token tq
         f32x4 s = {0.0f, 0.0f, 0.0f, 0.0f};
         if constexpr (BF16) {
@@ -748,6 +751,31 @@ __global__ __launch_bounds__(512) void k_prefill_attn(AttnParams p) {
     }
     l += __shfl_xor(l, 16);
     l += __shfl_xor(l, 32);
+    if (PW > 1) {
+        // the parts of a head join in LDS, [part - 1][head]: DT x 64 lanes of
+        // sums, then m and l; part 0 adds them in order
+        extern __shared__ float lds[];
+        constexpr int kPart = DT * 256 + 128;
+        if (part > 0) {
+            float* d = lds + ((part - 1) * G + hd) * kPart;
+#pragma unroll
+            for (int i = 0; i < DT; ++i) *reinterpret_cast<f32x4*>(d + i * 256 + lane * 4) = o[i];
+            d[DT * 256 + lane] = m;
+            d[DT * 256 + 64 + lane] = l;
+        }
+        __syncthreads();
+        if (part > 0) return;
+        for (int w = 1; w < PW; ++w) {
+            const float* d = lds + ((w - 1) * G + hd) * kPart;
+            const float mw = d[DT * 256 + lane], lw = d[DT * 256 + 64 + lane];
+            const float mn = fmaxf(m, mw);  // (part 0 has position 0, which every token sees)
+            const float a0 = expf(m - mn), a1 = mw == -INFINITY ? 0.0f : expf(mw - mn);
+#pragma unroll
+            for (int i = 0; i < DT; ++i) o[i] = o[i] * a0 + *reinterpret_cast<const f32x4*>(d + i * 256 + lane * 4) * a1;
+            l = l * a0 + lw * a1;
+            m = mn;
+        }
+    }
     if (S > 1) {  // the split's partial: unnormalised sums, m, l
         if (tq < T) {
 #pragma unroll
@@ -779,8 +807,16 @@ __global__ __launch_bounds__(512) void k_prefill_attn(AttnParams p) {
 template <int HD, bool BF16>
 static void launch_prefill_t(const AttnParams& p, hipStream_t st) {
     hipLaunchKernelGGL((k_qk_rope_cache<HD, BF16>), dim3(p.n_heads + 2 * p.n_kv, p.T), dim3(64), 0, st, p);
-    hipLaunchKernelGGL((k_prefill_attn<HD, BF16>), dim3((p.T + 15) / 16, p.n_kv),
-                       dim3(64 * (p.n_heads / p.n_kv)), 0, st, p);
+    // 8 waves per workgroup: with up to 2 q heads per kv head, or too few (head,
+    // tile) pairs for 2 waves on each SIMD, several waves share a head's blocks of
+    // positions (16 heads over 8, 301 tokens behind 77: float32 cache 53 -> 34 us
+    // with the prologue, bf16 29 -> 21; 2048 behind 600, bf16, 218 -> 196; 32 heads
+    // over 8, 512 tokens, 40 -> 37).  Otherwise one wave per head (32 over 8, 1024
+    // tokens: 98 us, 101 with two).
+    const int G = p.n_heads / p.n_kv, tiles = (p.T + 15) / 16;
+    const int PW = G <= 2 || tiles * p.n_heads < 2048 ? max(1, 8 / G) : 1;
+    hipLaunchKernelGGL((k_prefill_attn<HD, BF16>), dim3(tiles, p.n_kv), dim3(64 * G * PW),
+                       (size_t)(PW - 1) * G * (HD / 16 * 256 + 128) * 4, st, p);
 }
 
 int launch_prefill_attn(const AttnParams& p, hipStream_t st) {

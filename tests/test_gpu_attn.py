@@ -605,3 +605,30 @@ def test_prefill_attention_equals_batch_and_rejects_bad_blocks():
     assert L.rv12_prefill_attn_workspace_bytes(ctypes.byref(a), T) == T * H * HD * 4
     rc = L.rv12_prefill_rope_attn(ctypes.byref(a), T, None, None, None, None, None, None, None, None, None, 0, None)
     assert rc == _lib.RV12_E_NULL
+
+
+@pytest.mark.parametrize("H,KV,HD", [(8, 8, 64), (16, 8, 128), (32, 8, 128)])
+@pytest.mark.parametrize("T,p0", [(1, 0), (17, 0), (33, 5), (100, 60)])
+def test_prefill_attention_with_more_waves_than_blocks(H, KV, HD, T, p0):
+    """Several waves per head over few positions: parts without a block, with
+    blocks that a token does not see, and a last part that has the token's own
+    position; both cache types against float64 at the float32 bound of the
+    longest sums (head_dim products, then the positions)."""
+    from ai_amd.attn import RopeAttn
+    dev = "cuda"
+    g = torch.Generator(device=dev).manual_seed(T + H)
+    for dt in (torch.float32, torch.bfloat16):
+        maxt = p0 + T + 3
+        qkv = torch.randn(T, (H + 2 * KV) * HD, device=dev, generator=g)
+        one = torch.ones(HD, device=dev)
+        inv = torch.zeros(HD // 2, device=dev)  # no rotation: q is its RMSNorm
+        kc = torch.randn(KV, maxt, HD, device=dev, generator=g).to(dt)
+        vc = torch.randn(KV, maxt, HD, device=dev, generator=g).to(dt)
+        out = torch.empty(T, H * HD, device=dev)
+        RopeAttn(H, KV, HD, maxt, dt, 1e-6, dev).prefill(qkv, one, one, inv, torch.tensor([p0], device=dev), kc, vc, out, T)
+        q = qkv.view(T, H + 2 * KV, HD)[:, :H].double()
+        q = q / torch.sqrt((q * q).mean(-1, keepdim=True) + 1e-6)
+        ref = _prefill_ref(q, kc, vc, p0, T, H, KV, HD)
+        vmax = float(vc[:, :p0 + T].float().abs().max())
+        tol = (HD + p0 + T) * 2.0 ** -23 * HD ** 0.5 * vmax  # |score| <= sqrt(HD) |k| bound folded into one factor
+        assert float((out - ref).abs().max()) <= tol, (dt, float((out - ref).abs().max()), tol)
