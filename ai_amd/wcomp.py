@@ -39,11 +39,13 @@ _SK = {}   # (N, device) -> workspace tensor (split-K partial sums)
 
 
 def _ptr(t):
-    return None if t is None else ctypes.c_void_p(t.data_ptr())
+    return None if t is None else t.data_ptr()  # (the argument types make it a pointer)
 
 
 def _stream(dev):
-    return ctypes.c_void_p(torch.cuda.current_stream(dev).cuda_stream)
+    if dev.index is None:
+        return torch.cuda.current_stream(dev).cuda_stream
+    return torch._C._cuda_getCurrentRawStream(dev.index)  # the same without the Stream object: 2 us less
 
 
 def _need_cuda(t, what):
@@ -339,10 +341,17 @@ def _sk_buf(N, S, dev, K=None, T=16, cfg=None):
     every batch size; a buffer that must grow is retired, not freed, because a
     captured HIP graph may still hold its address (the retired ones go with
     _SK when the caches are cleared)."""
-    L = lib()
     K = int(K or 32 * max(S, 1))
-    need = max(L.rv12_launch_workspace_bytes(int(N), K, int(T), None if cfg is None else ctypes.byref(cfg)),
-               L.rv12_workspace_bytes(int(N), K, 16, 0))
+    return _sk_get(N, dev, _sk_need(int(N), K, int(T), cfg))
+
+
+def _sk_need(N, K, T, cfg):
+    L = lib()
+    return max(L.rv12_launch_workspace_bytes(N, K, T, None if cfg is None else ctypes.byref(cfg)),
+               L.rv12_workspace_bytes(N, K, 16, 0))
+
+
+def _sk_get(N, dev, need):
     k = (N, str(dev))
     if k not in _SK or _SK[k].numel() < need:
         if k in _SK:
@@ -357,6 +366,24 @@ def clear_caches():
     _SK.clear()
     _HEAD_WS.clear()
     _SK_RETIRED.clear()
+
+
+_RESOLVED = {}  # (N, K, T, BN, w, S) -> (validated Launch, workspace bytes), plain numbers both; at most 4096
+_RESOLVED_MAX = 4096
+
+
+def _resolved(N, K, T, BN, w, S):
+    """The launch of a linear and its workspace: three calls into the library
+    that depend on these six numbers alone.  An invalid one raises each time."""
+    key = (N, K, T, BN, w, S)
+    r = _RESOLVED.get(key)
+    if r is None:
+        cfg = _launch(BN, w, S, T)
+        launch_shape(N, K, T, cfg)  # validates the configuration (ValueError)
+        if len(_RESOLVED) >= _RESOLVED_MAX:
+            _RESOLVED.clear()
+        r = _RESOLVED[key] = (cfg, _sk_need(N, K, T, cfg))
+    return r
 
 
 def _linear(x, c, y, mode, T, BN, w, S, lnw, eps, where):
@@ -377,9 +404,8 @@ def _linear(x, c, y, mode, T, BN, w, S, lnw, eps, where):
         if lnw.dtype != torch.bfloat16 or lnw.numel() < K or not lnw.is_contiguous():
             raise ValueError(f"{where}: lnw must be a contiguous bf16 vector of K entries")
     m = _matrix(c)
-    cfg = _launch(BN, w, S, T)
-    launch_shape(N, K, T, cfg)  # validates the configuration (ValueError)
-    ws = _sk_buf(N, 0, x.device, K, T, cfg)
+    cfg, need = _resolved(N, K, T, BN, w, S)
+    ws = _sk_get(N, x.device, need)
     rc = lib().rv12_gemm(ctypes.byref(m), _ptr(x), _ptr(y), int(T), _ptr(lnw), float(eps), int(mode),
                          ctypes.byref(cfg), _ptr(ws), ws.numel(), _stream(x.device))
     check(rc, where)
