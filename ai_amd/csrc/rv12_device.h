@@ -144,21 +144,28 @@ __device__ __forceinline__ void split3(const float (&v)[8], u32x4& hi, u32x4& mi
     lo = u32x4{l[0] | l[1] << 16, l[2] | l[3] << 16, l[4] | l[5] << 16, l[6] | l[7] << 16};
 }
 
-// split 8 values into two float16x8 parts, hi + lo = v to 22 bits (a residual
-// below 2^-14 loses what is below 2^-24)
+// split 8 values below 2^15 into two float16x8 parts, hi + lo 2^-11 = v: to
+// 2^-23 of v for |v| >= 2^-13, to 2^-36 below (lo is a subnormal there).  The
+// products take hi with the weights scaled up by 2^11 (f16_up11), lo with the
+// weights as they are.
 __device__ __forceinline__ void split2_f16(const float (&v)[8], u32x4& hi, u32x4& lo) {
     uint32_t h[8], l[8];
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
         const _Float16 a = (_Float16)v[e];
         h[e] = (uint32_t)__builtin_bit_cast(uint16_t, a);
-        l[e] = (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)(v[e] - (float)a));
+        l[e] = (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)((v[e] - (float)a) * 2048.0f));
     }
     hi = u32x4{h[0] | h[1] << 16, h[2] | h[3] << 16, h[4] | h[5] << 16, h[6] | h[7] << 16};
     lo = u32x4{l[0] | l[1] << 16, l[2] | l[3] << 16, l[4] | l[5] << 16, l[6] | l[7] << 16};
 }
 
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+
+// eight float16 weights times 2^11, exactly (their exponent fields end at 15)
+__device__ __forceinline__ u32x4 f16_up11(u32x4 a) {
+    return __builtin_bit_cast(u32x4, __builtin_bit_cast(f16x8, a) * (_Float16)2048.0f);
+}
 
 // one v_mfma_f32_16x16x32_f16 (the lane layout of the bf16 one)
 __device__ __forceinline__ f32x4 mfma_f16(u32x4 a, u32x4 b, f32x4 c) {

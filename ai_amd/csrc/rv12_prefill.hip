@@ -16,18 +16,21 @@
 //      l: token l%16, k = 8(l/16) + 0..7), and x' itself in fp32, transposed
 //      (column-major over the padded tokens).  Token rows past T are zeros.
 //   2. k_prefill_mm: a 12-bit weight is exactly a float16 (4 exponent bits, 7
-//      of mantissa), so x' needs two float16 parts (22 bits) and two MFMAs per
-//      tile where three bf16 parts (24 bits) took three; the sums pass from
-//      the matrix core's accumulators to fp32 ones every kPfChunk steps and come
-//      out closer to 64 bits than before (24576 x 4096 over 2048 tokens:
-//      relative error 7.0e-7 -> 2.3e-7; 1024 x 3072 over 301: 1.95e-7 ->
-//      1.79e-7).  A tile with a token whose values the float16 parts would not
-//      hold (see tok_exp) keeps the three bf16 parts, and so does a call that
-//      asks for them (parts = 3): the prompt's qkv, whose keys and values are
-//      rounded into the cache and must stay, bit for bit, what earlier prompts
-//      left there (with two parts one in 10^4 bf16 entries falls on the other
-//      side of its rounding; the three parts cost the Qwen3-8B layer over 2048
-//      tokens about 40 us of 2036).
+//      of mantissa), so x' goes in two float16 parts (23 bits) with two MFMAs per
+//      tile where three bf16 parts (24 bits) took three.  The second part is kept
+//      2^11 larger, and the first meets the weights times 2^11 (they leave half of
+//      float16's exponents free): the parts hold a value 2^28 below its token's
+//      largest as well as the largest (2^17 without, for 2 % less time).  The sums
+//      pass from the matrix core's accumulators to fp32 ones every kPfChunk steps
+//      and come out closer to 64 bits than three parts in one accumulator (8192 x
+//      K over 1024 tokens, relative error, K = 512, 4096, 17408: 2.1e-7, 2.2e-7,
+//      2.5e-7 against 2.4e-7, 7.0e-7, 1.5e-6).  A tile with a token whose values
+//      the float16 parts would not hold (see tok_exp) keeps the three bf16 parts,
+//      and so does a call that asks for them (parts = 3): the prompt's qkv, whose
+//      keys and values are rounded into the cache and must stay, bit for bit, what
+//      earlier prompts left there (with two parts one in 10^4 bf16 entries falls
+//      on the other side of its rounding; the three parts cost the Qwen3-8B layer
+//      over 2048 tokens about 40 us of 2036).
 //      Workgroup = 256 rows x 128 tokens, 8 waves of 64 rows x 64 tokens.  Per
 //      32-column step the workgroup's 16 row blocks' Q16 tiles and the B parts
 //      go from memory straight into a ring of LDS slots (buffer loads with the
@@ -42,6 +45,7 @@
 //      product, took 3590 us, but leave no registers for the second sums:
 //      their error stays at 5.9e-7.)
 #include <hip/hip_runtime.h>
+#include <limits.h>
 #include <stdint.h>
 
 #include "rv12_device.h"
@@ -132,16 +136,23 @@ __device__ __forceinline__ void prefill_xprime(const float* xr, int K, int k, bo
     }
 }
 
-// A token's activation class, E = e << 1 | wide: e the largest exponent of
-// its finite nonzero |x'| (-1000: none), wide where the float16 split would
-// hold fewer bits of it than the float32 sums keep.  The float16 parts are of
-// x' 2^(15 - e): 22 bits of each value, and nothing below 2^-39 of the largest.
-// Where the mean exponent of the token's nonzero values is at least e - 14, the
-// root mean square of x' is at least 2^-15 of the largest (the geometric mean
-// is below it), so the second part is below 2^-24 of it; other tokens (a few
-// huge values among tiny ones) are wide and keep the three bf16 parts, as
-// does every token of their tile.
-constexpr int kF16MeanBelow = 14;
+// A token's activation class, E = e << 1 | wide: e the exponent of its largest
+// finite |x'| (below B = 2^e; -1000: all zeros), wide where the float16 parts
+// would hold less of it than float32 sums do; such a token keeps three bf16
+// parts, and so does every token of its tile.  The float16 parts are of
+// x' 2^(15 - e): every |x'| >= 2^-28 B to 2^-23 of itself, a smaller one to 2^-51 B.
+// So a token without a nonzero value below 2^-28 B is not wide.  One with such
+// values must bear rows whose weights lie on them alone.  A row keeps in its tiles
+// the 15 exponents that most of its weights have: at least K / 18 weights (18
+// windows cover the 256 exponents), less than 2^15 apart.  With at most K / 36
+// columns at or below 2^-16 B (zeros included), K / 36 of those weights are on
+// larger ones, and n small values add an error of less than
+// n 2^15 2^-51 / ((K / 36) 2^-16) of sum |w||x'|: below 2^-23 for n <= K / 512.
+// (Base 0 is the exception: its window holds the zeros, its weights are
+// below 2^-112.)  Of 1024 tokens of 12288 columns silu(g) u with normal g and u, 8
+// have a value below 2^-28 B, one each, none more than 58 columns below 2^-16 B:
+// none is wide.  One with half its columns 2^29 below the others is.
+constexpr int kF16Exact = 28, kF16Floor = 16;  // exponents below B
 __device__ __forceinline__ int tok_exp(int E) { return E >> 1; }
 __device__ __forceinline__ int scale_f16(int E) { return tok_exp(E) < -500 ? 0 : 15 - tok_exp(E); }
 __device__ __forceinline__ int scale_bf16(int E) {
@@ -159,19 +170,20 @@ __device__ __forceinline__ int wide_lanes(const int* __restrict__ E, int t0, int
 }
 
 // 1a. k_prefill_stats: one wave per token (4 per workgroup, a grid over the
-// padded tokens): the largest exponent of |x'|, the sum of its exponents and,
-// with RMS, the sum of squares of x 2^-32, lane l over columns 8 l + 512 i,
-// reduced across the wave in a fixed order; writes the token's E and rs_t.
+// padded tokens): the largest and smallest exponent of the nonzero x' and, with
+// RMS, the sum of squares of x 2^-32, lane l over columns 8 l + 512 i, reduced
+// across the wave in a fixed order; where the smallest asks for them, the counts
+// of small columns in a second pass over the row; writes the token's E and rs_t.
 constexpr int kPsThreads = 256;
 __global__ __launch_bounds__(kPsThreads) void k_prefill_stats(const float* __restrict__ x, int T, int K, int xs,
                                                               int m2, const uint16_t* __restrict__ lnw, float eps,
                                                               int* __restrict__ E, float* __restrict__ R) {
     const int lane = threadIdx.x & 63;
     const int t = blockIdx.x * (kPsThreads / 64) + (threadIdx.x >> 6);
-    int e = -1000, cnt = 0, es = 0;  // |es| <= 2^20 columns x 149
+    uint32_t hib = 0, lob = 0xFFFFFFFFu;  // magnitudes as bits: the largest finite, the smallest nonzero less one
     float sq = 0.0f;
+    const float* xr = x + (int64_t)t * xs;
     if (t < T) {
-        const float* xr = x + (int64_t)t * xs;
         for (int k = lane * 8; k < K; k += 512) {
             float v[8];
             prefill_xprime(xr, K, k, m2 != 0, nullptr, v);
@@ -188,23 +200,57 @@ __global__ __launch_bounds__(kPsThreads) void k_prefill_stats(const float* __res
             }
 #pragma unroll
             for (int i = 0; i < 8; ++i) {
-                const int ei = exp_or_min(v[i]);
-                const bool ok = ei > -1000;
-                e = max(e, ei);
-                cnt += ok ? 1 : 0;
-                es += ok ? ei : 0;
+                const uint32_t b = __float_as_uint(v[i]) & 0x7FFFFFFFu;
+                hib = max(hib, b < 0x7F800000u ? b : 0u);
+                lob = min(lob, b - 1);
             }
         }
     }
 #pragma unroll
     for (int o = 32; o >= 1; o >>= 1) {
-        e = max(e, __shfl_xor(e, o));
-        cnt += __shfl_xor(cnt, o);
-        es += __shfl_xor(es, o);
+        hib = max(hib, (uint32_t)__shfl_xor((int)hib, o));
+        lob = min(lob, (uint32_t)__shfl_xor((int)lob, o));
         sq += __shfl_xor(sq, o);
     }
+    const int e = exp_or_min(__uint_as_float(hib));
+    // a row with small values: all the workgroup's waves count them (one wave's second
+    // pass over 12288 columns would end 13 us after the others)
+    constexpr int kWaves = kPsThreads / 64;
+    __shared__ int top[kWaves], cnt[kWaves][2];  // the row's e, or INT_MAX without small values; counts
+    const int wave = threadIdx.x >> 6;
     if (lane == 0) {
-        const bool wide = (int64_t)es < (int64_t)cnt * (e - kF16MeanBelow);
+        top[wave] = hib && exp_or_min(__uint_as_float(lob + 1)) <= e - kF16Exact ? e : INT_MAX;
+        cnt[wave][0] = cnt[wave][1] = 0;
+    }
+    __syncthreads();
+    for (int w = 0; w < kWaves; ++w) {
+        const int ew = top[w];
+        if (ew == INT_MAX) continue;
+        const float* row = x + (int64_t)(t - wave + w) * xs;
+        int tiny = 0, small = 0;
+        for (int k = threadIdx.x * 8; k < K; k += kPsThreads * 8) {
+            float v[8];
+            prefill_xprime(row, K, k, m2 != 0, lnw, v);
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {  // (frexp exponents: |x'| < 2^ei)
+                const int ei = exp_or_min(v[i]);
+                tiny += ei > -1000 && ei <= ew - kF16Exact ? 1 : 0;
+                small += v[i] == 0.0f || (ei > -1000 && ei <= ew - kF16Floor) ? 1 : 0;
+            }
+        }
+#pragma unroll
+        for (int o = 32; o >= 1; o >>= 1) {
+            tiny += __shfl_xor(tiny, o);
+            small += __shfl_xor(small, o);
+        }
+        if (lane == 0) {
+            atomicAdd(&cnt[w][0], tiny);
+            atomicAdd(&cnt[w][1], small);
+        }
+    }
+    __syncthreads();
+    if (lane == 0) {
+        const bool wide = cnt[wave][0] > K / 512 || cnt[wave][1] > K / 36;
         E[t] = e * 2 + (wide ? 1 : 0);
         if (lnw) R[t] = rms_scale(sq, K, eps);
     }
@@ -246,8 +292,8 @@ __global__ __launch_bounds__(kPpThreads) void k_prefill_parts(const float* __res
     } else {
         split2_f16(v, hi, lo);
         u32x4* d = blk + (int64_t)s * 128 + l;
-        d[0] = hi;
-        d[64] = lo;
+        d[0] = lo;
+        d[64] = hi;
     }
 }
 
@@ -370,7 +416,7 @@ __global__ __launch_bounds__(kPfThreads) void k_prefill_mm(const uint32_t* __res
         __builtin_amdgcn_s_waitcnt(waitcnt_vm(kPfWait2));
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
-        u32x4 a[2][kPfWB], fb[W];
+        u32x4 a[2][kPfWB], up[kPfWB], fb[W];  // up: the step's weights times 2^11, for the hi parts
 #pragma unroll
         for (int b = 0; b < kPfWB; ++b) {
             const u32x3 r = read_a(0, b);
@@ -407,10 +453,12 @@ __global__ __launch_bounds__(kPfThreads) void k_prefill_mm(const uint32_t* __res
 #pragma unroll
                     for (int i = 0; i < kFrags; ++i) {
                         if (i < kPfOps2) load_op(i, fill, s0 + u + kPfRing2 - 1);
-                        if (i < kPfWB) raw[i] = read_a(nxt, i);
+                        if (i >= 1 && i - 1 < kPfWB) raw[i - 1] = read_a(nxt, i - 1);
                         const u32x4 bf = fb[i % W];
 #pragma unroll
-                        for (int b = 0; b < kPfWB; ++b) acc[b][i % kPfWT] = mfma_f16(a[u][b], bf, acc[b][i % kPfWT]);
+                        for (int b = 0; b < kPfWB; ++b)
+                            acc[b][i % kPfWT] = mfma_f16(i < kPfWT ? a[u][b] : up[b], bf, acc[b][i % kPfWT]);
+                        if (i < kPfWB) up[i] = f16_up11(a[u][i]);
                         fb[i % W] = i + W < kFrags ? read_b(cur, i + W) : read_b(nxt, i + W - kFrags);
                         if (i >= kFrags - kPfWB) {
                             const int b = i - (kFrags - kPfWB);
@@ -555,7 +603,7 @@ __global__ __launch_bounds__(kPfThreads) void k_prefill_mm(const uint32_t* __res
 #pragma unroll
     for (int c = 0; c < kPfWT; ++c) {
         const int et = E[min((tbw + c) * 16 + jj, T - 1)];
-        const int pt = wide ? scale_bf16(et) : scale_f16(et) + kF16WeightExp;
+        const int pt = wide ? scale_bf16(et) : scale_f16(et) + kF16WeightExp + 11;
 #pragma unroll
         for (int b = 0; b < kPfWB; ++b)
 #pragma unroll

@@ -10,11 +10,11 @@ dense GEMM, instead of passes of 16 tokens through the fused decode-linear.
 
 MI355X form of `matrix`: one fused kernel chain in librv12
 (rv12_prefill_linear): the fp32 activations of all prompt tokens are split
-once, after an exact per-token power-of-two scale, into two float16 parts (22
-significand bits; a 12-bit weight is exactly a float16), or into three bf16
-parts (24 bits, the reference's own split for bf16 matrix units,
-ramvi/engine/ramvi_engine/kernels/wcomp.py:130-140) where a token's values
-spread over more exponents than float16 holds, and a hand-written MFMA GEMM
+once, after an exact per-token power-of-two scale, into two float16 parts (23
+significand bits down to 2^-28 of the token's largest value; a 12-bit weight is
+exactly a float16), or into three bf16 parts (24 bits, the reference's own split
+for bf16 matrix units, ramvi/engine/ramvi_engine/kernels/wcomp.py:130-140) where
+so many of a token's values are smaller that a row could live on them, and a hand-written MFMA GEMM
 reads each weight once in its 12-bit packed form (the Q16 tiles are the
 MFMA's A operand), accumulates in fp32 and adds the
 exceptions; no wider copy of W is ever written.  The reference computes the

@@ -272,6 +272,78 @@ def test_tokens_over_many_exponents(N, T, big):
     assert np.all(err <= 4 * (K + 8) * 2.0 ** -24 * mag + 1e-30), float((err / mag).max())
 
 
+def _on_gpu(bits):
+    return torch.from_numpy(bits.view(np.int16)).view(torch.bfloat16).cuda()
+
+
+@pytest.mark.parametrize("K,low", [(32, 17), (64, 34), (480, 14), (544, 300), (4096, 200), (4096, 2200)])
+@pytest.mark.parametrize("drop", [14, 20, 25, 28, 36, 60])
+def test_tokens_of_two_levels(K, low, drop):
+    """`low` columns 2^drop below the others, in every third token, and rows with
+    weights on those columns alone (kept in the tiles where they are more than the
+    zeros).  The norm of a token's error over the rows stays below
+    sqrt(K) 2^-24 of its output's, the random walk of a float32 sum of K products,
+    plus 2^-23 for the split of the activations, for the rows of either kind; so
+    does a token of one level in the same tile."""
+    from ai_amd import prefill, wcomp
+    rng = np.random.default_rng(K + low + drop)
+    N, T = 512, 140
+    cols = rng.choice(K, low, replace=False)
+    w = (rng.standard_normal((N, K)) * 0.02).astype(np.float32)
+    w = np.copysign(np.maximum(np.abs(w), 1e-3), w)
+    rest = np.setdiff1d(np.arange(K), cols)
+    w[::2, rest] = 0
+    bits = codec.f32_to_bf16_rne(w)
+    x = rng.standard_normal((T, K)).astype(np.float32)
+    x[::3, cols] *= np.float32(2.0) ** -drop
+    y = torch.zeros(T, N, device="cuda")
+    prefill.matrix(torch.from_numpy(x).cuda(), wcomp.compress(_on_gpu(bits), CH=32), y)
+    want = x.astype(np.float64) @ codec.bf16_to_f32(bits).astype(np.float64).T
+    err = y.cpu().numpy() - want
+    for rows in (slice(0, N, 2), slice(1, N, 2)):
+        rel = np.linalg.norm(err[:, rows], axis=1) / np.linalg.norm(want[:, rows], axis=1)
+        print("K", K, "low", low, "drop", drop, "rel", float(rel.max()), flush=True)
+        assert rel.max() <= K ** 0.5 * 2.0 ** -24 + 2.0 ** -23, (float(rel.max()), int(rel.argmax()))
+
+
+def test_sums_over_chunks_keep_their_accuracy():
+    """K = 4096 unsplit: the norm of the error stays below 4e-7 of the output's
+    (2.3e-7 measured; 5.9e-7 without the float32 sums over chunks of steps, 5e-5
+    without the activations' second part)."""
+    from ai_amd import _lib, prefill, wcomp
+    N, K, T = 8192, 4096, 1024
+    g = torch.Generator(device="cuda").manual_seed(5)
+    assert _lib.lib().rv12_prefill_workspace_bytes(N, K, T) == T * K * 10 + T * 8  # no K split
+    w = (torch.randn(N, K, device="cuda", generator=g) * 0.02).bfloat16()
+    x = torch.randn(T, K, device="cuda", generator=g)
+    y = torch.zeros(T, N, device="cuda")
+    prefill.matrix(x, wcomp.compress(w), y)
+    want = x.double() @ w.double().t()
+    rel = float((y.double() - want).norm() / want.norm())
+    assert rel <= 4e-7, rel
+
+
+def test_three_parts_hold_24_bits():
+    """parts = 3: an activation of 24 significant bits times a power of two comes
+    out exactly.  (Two float16 parts hold 23: half of these lose their last.)"""
+    from ai_amd import prefill, wcomp
+    rng = np.random.default_rng(24)
+    N, K, T = 64, 96, 200
+    bits = codec.f32_to_bf16_rne((2.0 ** rng.integers(-9, -3, (N, K)) * rng.choice([-1, 1], (N, K))).astype(np.float32))
+    x = np.zeros((T, K), np.float32)
+    at = rng.integers(0, K, T)
+    x[np.arange(T), at] = (rng.integers(1 << 22, 1 << 23, T) * 2 + 1).astype(np.float32)
+    v = x[np.arange(T), at] / np.float32(2.0 ** 9)
+    hi = v.astype(np.float16).astype(np.float32)
+    two = hi + ((v - hi) * np.float32(2048)).astype(np.float16).astype(np.float32) / np.float32(2048)
+    assert np.count_nonzero(two != v) > T // 4  # two parts could not pass
+    c = wcomp.compress(_on_gpu(bits), CH=32)
+    y = torch.zeros(T, N, device="cuda")
+    prefill._linear(torch.from_numpy(x).cuda(), c, y, 0, parts=3)
+    want = x[np.arange(T), at][:, None] * codec.bf16_to_f32(bits).T[at]
+    assert np.array_equal(y.cpu().numpy(), want)
+
+
 @pytest.mark.parametrize("T,K", [(17, 160), (300, 512), (130, 1056)])
 def test_three_parts_on_request(T, K):
     """parts = 3: the linear whose outputs are rounded into the caches; steps off
