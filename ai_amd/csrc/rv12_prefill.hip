@@ -24,13 +24,13 @@
 //      pass from the matrix core's accumulators to fp32 ones every kPfChunk steps
 //      and come out closer to 64 bits than three parts in one accumulator (8192 x
 //      K over 1024 tokens, relative error, K = 512, 4096, 17408: 2.1e-7, 2.2e-7,
-//      2.5e-7 against 2.4e-7, 7.0e-7, 1.5e-6).  A tile with a token whose values
-//      the float16 parts would not hold (see tok_exp) keeps the three bf16 parts,
-//      and so does a call that asks for them (parts = 3): the prompt's qkv, whose
-//      keys and values are rounded into the cache and must stay, bit for bit, what
-//      earlier prompts left there (with two parts one in 10^4 bf16 entries falls
-//      on the other side of its rounding; the three parts cost the Qwen3-8B layer
-//      over 2048 tokens about 40 us of 2036).
+//      2.5e-7 against 2.4e-7, 7.0e-7, 1.5e-6).  A token whose values the float16
+//      parts would not hold (see tok_exp) keeps the three bf16 parts, whatever the
+//      others of its tile do, and so do all tokens of a call that asks for them
+//      (parts = 3): the prompt's qkv, whose keys and values are rounded into the
+//      cache and must stay, bit for bit, what earlier prompts left there (with two
+//      parts one in 10^4 bf16 entries falls on the other side of its rounding; the
+//      three parts cost the Qwen3-8B layer over 2048 tokens about 40 us of 2036).
 //      Workgroup = 256 rows x 128 tokens, 8 waves of 64 rows x 64 tokens.  Per
 //      32-column step the workgroup's 16 row blocks' Q16 tiles and the B parts
 //      go from memory straight into a ring of LDS slots (buffer loads with the
@@ -47,6 +47,8 @@
 #include <hip/hip_runtime.h>
 #include <limits.h>
 #include <stdint.h>
+
+#include <type_traits>
 
 #include "rv12_device.h"
 #include "rv12_internal.h"
@@ -139,7 +141,7 @@ __device__ __forceinline__ void prefill_xprime(const float* xr, int K, int k, bo
 // A token's activation class, E = e << 1 | wide: e the exponent of its largest
 // finite |x'| (below B = 2^e; -1000: all zeros), wide where the float16 parts
 // would hold less of it than float32 sums do; such a token keeps three bf16
-// parts, and so does every token of its tile.  The float16 parts are of
+// parts.  The float16 parts are of
 // x' 2^(15 - e): every |x'| >= 2^-28 B to 2^-23 of itself, a smaller one to 2^-51 B.
 // So a token without a nonzero value below 2^-28 B is not wide.  One with such
 // values must bear rows whose weights lie on them alone.  A row keeps in its tiles
@@ -160,13 +162,10 @@ __device__ __forceinline__ int scale_bf16(int E) {
     return (e >= -39 && e <= kXRangeHi) ? kXScaleExp : slow_scale_exp(e);
 }
 
-// any of the tile's tokens t0 .. t0 + 127 below T is wide (t0 < T): the lanes'
-// part of the answer, a ballot of bit 0 away from the whole
-__device__ __forceinline__ int wide_lanes(const int* __restrict__ E, int t0, int T) {
-    int any = 0;
-#pragma unroll
-    for (int i = 0; i < kPfTokens; i += 64) any |= E[min(t0 + i + (int)(threadIdx.x & 63), T - 1)];
-    return any;
+// which of the tokens t0 .. t0 + 63 are wide (t0 < T; past T: as the last one)
+__device__ __forceinline__ uint64_t wide_mask(int E) { return __ballot(E & 1); }
+__device__ __forceinline__ int class_of(const int* __restrict__ E, int t0, int T) {
+    return E[min(t0 + (int)(threadIdx.x & 63), T - 1)];
 }
 
 // 1a. k_prefill_stats: one wave per token (4 per workgroup, a grid over the
@@ -260,7 +259,9 @@ __global__ __launch_bounds__(kPsThreads) void k_prefill_stats(const float* __res
 // thread (token tok, 8-column group k8): x' (prologue applied) of token t at
 // columns kc .. kc + 7 written transposed (per column, 32 consecutive tokens:
 // full 128-byte lines), then its scaled parts in B-operand lane order: two of
-// float16, or three of bf16 where a token of the GEMM's 128-token tile is wide.  Tokens past T are zeros.
+// float16 (the second first), or three of bf16 for a wide token.  A token block's
+// region holds the first two parts of its steps, then the third ones (unwritten,
+// and unused, for the lanes of tokens that have two).  Tokens past T are zeros.
 constexpr int kPpThreads = 256;
 __global__ __launch_bounds__(kPpThreads) void k_prefill_parts(const float* __restrict__ x, int T, int K, int xs,
                                                               int m2, const uint16_t* __restrict__ lnw,
@@ -272,29 +273,23 @@ __global__ __launch_bounds__(kPpThreads) void k_prefill_parts(const float* __res
     const int nsteps = K >> 5;
     float v[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
     if (t < T && kc < K) prefill_xprime(x + (int64_t)t * xs, K, kc, m2 != 0, lnw, v);
-    const bool wide = parts == 3 || __ballot(wide_lanes(E, (int)(blockIdx.x * 32) / kPfTokens * kPfTokens, T) & 1) != 0;
     if (kc >= K) return;
     float* xc = xt + (int64_t)kc * tp + t;
 #pragma unroll
     for (int i = 0; i < 8; ++i) xc[(int64_t)i * tp] = v[i];
-    const int p = t < T ? (wide ? scale_bf16(E[t]) : scale_f16(E[t])) : 0;
+    const int et = t < T ? E[t] : 0;
+    const bool wide = parts == 3 || (et & 1);
+    const int p = t >= T ? 0 : wide ? scale_bf16(et) : scale_f16(et);
 #pragma unroll
     for (int i = 0; i < 8; ++i) v[i] = ldexpf(v[i], p);
     const int s = kc >> 5, l = ((kc & 31) >> 3) * 16 + (t & 15);  // step, lane of the operand
-    u32x4* blk = xb + (int64_t)(t >> 4) * nsteps * 192;
-    u32x4 hi, mid, lo;
-    if (wide) {
-        split3(v, hi, mid, lo);
-        u32x4* d = blk + (int64_t)s * 192 + l;
-        d[0] = hi;
-        d[64] = mid;
-        d[128] = lo;
-    } else {
-        split2_f16(v, hi, lo);
-        u32x4* d = blk + (int64_t)s * 128 + l;
-        d[0] = lo;
-        d[64] = hi;
-    }
+    u32x4* blk = xb + (int64_t)(t >> 4) * nsteps * 192 + l;
+    u32x4 d[3];
+    if (wide) split3(v, d[0], d[1], d[2]);
+    else split2_f16(v, d[1], d[0]);
+    blk[(int64_t)s * 128] = d[0];
+    blk[(int64_t)s * 128 + 64] = d[1];
+    if (wide) blk[(int64_t)nsteps * 128 + (int64_t)s * 64] = d[2];
 }
 
 // Workgroup i -> (row tile, token tile).  Workgroups are dispatched in order,
@@ -348,9 +343,9 @@ __global__ __launch_bounds__(kPfThreads) void k_prefill_mm(const uint32_t* __res
     const int64_t blk0 = (int64_t)rt * kPfRowBlocks + wr * kPfWB;  // this wave's first row block
     const int tb0 = tt * kPfTokBlocks;                            // the workgroup's first token block
     const uint32_t blk_bytes = (uint32_t)nsteps * kStepBytes;
-    // a wide token in the tile: the parts are three of bf16 (asked for here,
-    // answered after the first loads are on their way)
-    const int wl = wide_lanes(E, tb0 * 16, T);
+    // the classes of the tile's tokens (asked for here, answered after the first
+    // loads are on their way)
+    const int wl0 = class_of(E, tb0 * 16, T), wl1 = class_of(E, tb0 * 16 + 64, T);
     // the workgroup's A tiles: wave w loads row blocks 2w and 2w + 1 of the
     // workgroup through a descriptor over its valid row blocks (a row block
     // past N, or a step past the end through the 0-byte descriptor, reads
@@ -367,12 +362,6 @@ __global__ __launch_bounds__(kPfThreads) void k_prefill_mm(const uint32_t* __res
     const u32x4* xbw = xb + (int64_t)tb0 * nsteps * 192;
     const __amdgpu_buffer_rsrc_t rbx = make_rsrc(xbw, (uint32_t)kPfTokBlocks * nsteps * 192 * 16);
     const __amdgpu_buffer_rsrc_t rbnull = make_rsrc(xbw, 0u);
-
-    f32x4 acc[kPfWB][kPfWT];
-#pragma unroll
-    for (int b = 0; b < kPfWB; ++b)
-#pragma unroll
-        for (int c = 0; c < kPfWT; ++c) acc[b][c] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 
     constexpr int kFrags = 2 * kPfWT;
     constexpr int W = 4;  // B fragments in flight (8: the same within 1 %)
@@ -395,17 +384,32 @@ __global__ __launch_bounds__(kPfThreads) void k_prefill_mm(const uint32_t* __res
             load_lds16(in ? rbx : rbnull, d + kPfSlotA + wave * 64 + (i - kPfAPerWave) * kPfThreads,
                        boff[i - kPfAPerWave], (in ? s : 0) * 128 * 16);
     };
-    // steps 0 .. kPfRing2 - 2 into slots 0 .. (a wide tile starts over: what these
-    // loads bring is in bounds and unused)
+    // steps 0 .. kPfRing2 - 2 into slots 0 .. (a tile of wide tokens alone starts
+    // over: what these loads bring is in bounds and unused)
     if (parts == 2) {
 #pragma unroll
         for (int j = 0; j < kPfRing2 - 1; ++j)
 #pragma unroll
             for (int i = 0; i < kPfOps2; ++i) load_op(i, j * kPfSlot2, j);
     }
-    const bool wide = parts == 3 || __ballot(wl & 1) != 0;
+    // Two passes over a tile with tokens of both classes, each storing its own
+    // tokens' outputs (an MFMA's output column is its own token's alone: what the other
+    // class's bits give stays in columns that are not stored), so that a
+    // token's result is the same beside any others.  (24576 x 4096 over 2048
+    // tokens, of one class 824 and 1009 us: 862 with one wide token in one tile,
+    // 1246 with one in each, 1610 with one in 20; three parts for the whole tile
+    // took 1000 with any.)  Three parts: one pass.
+    const uint64_t w0 = parts == 3 ? ~0ull : wide_mask(wl0), w1 = parts == 3 ? ~0ull : wide_mask(wl1);
+    const uint64_t ww = wc ? w1 : w0;  // the wave's 64 tokens
+    auto tile_pass = [&](auto wide_c) {
+    constexpr bool wide = decltype(wide_c)::value;
+    f32x4 acc[kPfWB][kPfWT];
+#pragma unroll
+    for (int b = 0; b < kPfWB; ++b)
+#pragma unroll
+        for (int c = 0; c < kPfWT; ++c) acc[b][c] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 
-    if (!wide) {
+    if constexpr (!wide) {
         const int ra0 = wr * kPfWB * 64 + lane, rb0 = kPfSlotA + wc * kPfWT * 128 + lane;
         auto read_a = [&](int slot, int b) { return *reinterpret_cast<const u32x3*>(bs + slot + ra0 + b * 64); };
         // fragment i: part i / kPfWT of token block i % kPfWT, so that the products
@@ -486,28 +490,33 @@ __global__ __launch_bounds__(kPfThreads) void k_prefill_mm(const uint32_t* __res
 #pragma unroll
             for (int c = 0; c < kPfWT; ++c) acc[b][c] = sum[b][c];
     } else {
+        // the first loads have landed, and a first pass's LDS accesses are done
         asm volatile("" ::: "memory");
-        __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));
+        __builtin_amdgcn_s_waitcnt(waitcnt_vm_lgkm0(0));
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
-        int boff3[3];
+        int boff3[3], bstep3[3];
 #pragma unroll
         for (int j = 0; j < 3; ++j) {
-            const int idx = tid + j * kPfThreads;  // (token block, part, lane) of the step
-            boff3[j] = ((idx / 192) * nsteps * 192 + idx % 192) * 16;
+            const int ch = wave + j * kPfWaves, pt = ch % 3;  // (token block, part) of the step
+            boff3[j] = ((ch / 3 * 192 + (pt < 2 ? 0 : 128)) * nsteps + (pt & 1) * 64 + lane) * 16;
+            bstep3[j] = pt < 2 ? 128 * 16 : 64 * 16;
         }
+        int need = 0;  // the wave's token blocks with a wide token
+#pragma unroll
+        for (int c = 0; c < kPfWT; ++c) need |= (ww >> (16 * c) & 0xFFFF) != 0 ? 1 << c : 0;
         auto load_step = [&](int slot, int j) {  // step s_lo + j
             const int s = s_lo + j;
             const bool in = s < s_hi;
             const __amdgpu_buffer_rsrc_t ra = in ? rv : rnull, rb = in ? rbx : rbnull;
-            const int sa = (in ? s : 0) * kStepBytes, sb = (in ? s : 0) * 192 * 16;
+            const int sa = (in ? s : 0) * kStepBytes, sb = in ? s : 0;
             u32x4* d = bs + slot * kPfSlot3;
 #pragma unroll
             for (int i = 0; i < kPfAPerWave; ++i)
                 load_lds12(ra, d + (wave * kPfAPerWave + i) * 64, aoff[i], sa);
 #pragma unroll
             for (int j = 0; j < 3; ++j)
-                load_lds16(rb, d + kPfSlotA + wave * 64 + j * kPfThreads, boff3[j], sb);
+                load_lds16(rb, d + kPfSlotA + wave * 64 + j * kPfThreads, boff3[j], sb * bstep3[j]);
         };
         // this wave's fragments of the step in slot `slot`: its 4 row blocks' A
         // groups and 3 parts x 4 token blocks of B, part-major so the first
@@ -518,9 +527,10 @@ __global__ __launch_bounds__(kPfThreads) void k_prefill_mm(const uint32_t* __res
             for (int b = 0; b < kPfWB; ++b) fa[b] = *reinterpret_cast<const u32x3*>(d + (wr * kPfWB + b) * 64 + lane);
             const u32x4* src = d + kPfSlotA + wc * kPfWT * 192 + lane;
 #pragma unroll
-            for (int q = 0; q < 3; ++q)
+            for (int c = 0; c < kPfWT; ++c)
+                if (need >> c & 1)
 #pragma unroll
-                for (int c = 0; c < kPfWT; ++c) fb[q][c] = src[c * 192 + q * 64];
+                    for (int q = 0; q < 3; ++q) fb[q][c] = src[c * 192 + q * 64];
         };
         // steps 0-3 into slots 0-3, all landed; step 0's fragments read
 #pragma unroll
@@ -534,8 +544,9 @@ __global__ __launch_bounds__(kPfThreads) void k_prefill_mm(const uint32_t* __res
         read_frags(fa[0], fb[0], 0);
         // Step s: wait for this wave's loads of step s + 1 and its fragment reads
         // of step s; barrier; step s + 4 into slot s % 4; the fragments of step
-        // s + 1 read while the 48 MFMAs of step s run.  Whole rounds of the
-        // unroll: steps past the split read zeros and add nothing.
+        // s + 1 read while the 48 MFMAs of step s run (12 for each token block that
+        // has a wide token).  Whole rounds of the unroll: steps past the split read
+        // zeros and add nothing.
         for (int s0 = 0; s0 < s_hi - s_lo; s0 += kPfRing3) {
 #pragma unroll
             for (int u = 0; u < kPfRing3; ++u) {
@@ -555,11 +566,13 @@ __global__ __launch_bounds__(kPfThreads) void k_prefill_mm(const uint32_t* __res
                     a[b] = u32x4{pr[0], pr[1], pr[2], pr[3]};
                 }
 #pragma unroll
-                for (int q = 0; q < 3; ++q)
+                for (int c = 0; c < kPfWT; ++c) {
+                    if (!(need >> c & 1)) continue;
 #pragma unroll
-                    for (int b = 0; b < kPfWB; ++b)
+                    for (int q = 0; q < 3; ++q)
 #pragma unroll
-                        for (int c = 0; c < kPfWT; ++c) acc[b][c] = mfma(a[b], fb[u & 1][q][c], acc[b][c]);
+                        for (int b = 0; b < kPfWB; ++b) acc[b][c] = mfma(a[b], fb[u & 1][q][c], acc[b][c]);
+                }
             }
         }
     }
@@ -581,7 +594,7 @@ __global__ __launch_bounds__(kPfThreads) void k_prefill_mm(const uint32_t* __res
     const int64_t rlo = blk0 * 16;
     __builtin_amdgcn_s_barrier();  // the ring's LDS is the exception sums' from here
     asm volatile("" ::: "memory");
-    if (rlo >= N) return;
+    if (rlo >= N || (wide ? ww : ~ww) == 0) return;  // nothing of this pass to store
     const int32_t e_lo = rp[rlo], e_hi = rp[min(rlo + 16 * kPfWB, (int64_t)N)];
     const bool vec = (N & 3) == 0;  // y, part and rbase are 16-byte aligned
     int64_t nr[kPfWB];              // the lane's first row of each tile
@@ -696,7 +709,7 @@ __global__ __launch_bounds__(kPfThreads) void k_prefill_mm(const uint32_t* __res
             f32x4 v = acc[b][c];
             if constexpr (LN) v *= rs[c];
             if (add && S == 1) v = oy[b][c] + v;
-            if (tok[c] >= T) continue;
+            if (tok[c] >= T || (ww >> (16 * c + jj) & 1) != (wide ? 1 : 0)) continue;
             if (vec) {
                 if (nr[b] < N) *reinterpret_cast<f32x4*>(dst + nr[b]) = v;
             } else {
@@ -706,6 +719,9 @@ __global__ __launch_bounds__(kPfThreads) void k_prefill_mm(const uint32_t* __res
             }
         }
     }
+    };
+    if ((w0 & w1) != ~0ull) tile_pass(std::false_type{});
+    if ((w0 | w1) != 0) tile_pass(std::true_type{});
 }
 
 int prefill_tokens_padded(int T) { return (T + kPfTokens - 1) / kPfTokens * kPfTokens; }

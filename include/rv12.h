@@ -249,9 +249,10 @@ int rv12_gemm_static(const rv12_matrix* w, const float* x, float* y, int t, cons
  * x' is split per token, after an exact power-of-two scale, into two float16
  * parts: 23 significand bits of every value down to 2^-28 of the bound 2^e of the
  * token's largest, 2^-51 2^e of a smaller one; or into three bf16 parts (24 bits of
- * every value) in a tile with a token of more than k / 512 nonzero values below 2^-28 2^e,
- * or of any and more than k / 36 columns below 2^-16 2^e, whose small columns could
- * make up an output (given the row windows rv12_pack_plan chooses).  Every
+ * every value) where more than k / 512 nonzero values are below 2^-28 2^e, or any
+ * is and more than k / 36 columns are below 2^-16 2^e, so that small columns could
+ * make up an output (given the row windows rv12_pack_plan chooses).  A token's
+ * outputs depend on its own row and on t, on no other token.  Every
  * weight is read once in its 12-bit form, products and sums are fp32, the
  * exceptions are added in list order.  Where
  * the rows and tokens give too few workgroups to fill the GPU (few tokens, or

@@ -306,6 +306,32 @@ def test_tokens_of_two_levels(K, low, drop):
         assert rel.max() <= K ** 0.5 * 2.0 ** -24 + 2.0 ** -23, (float(rel.max()), int(rel.argmax()))
 
 
+@pytest.mark.parametrize("N,K,T", [(300, 256, 140), (301, 1056, 300), (22003, 160, 200)])
+@pytest.mark.parametrize("mode", [0, 1])
+def test_a_token_does_not_depend_on_its_neighbours(N, K, T, mode):
+    """The same token rows beside tokens of many exponents and without, K split and
+    unsplit, rows with exceptions, store and add: bit for bit the same outputs."""
+    from ai_amd import prefill, wcomp
+    rng = np.random.default_rng(N + K)
+    w = (rng.standard_normal((N, K)) * 0.02).astype(np.float32)
+    w.reshape(-1)[rng.choice(w.size, 200, replace=False)] = 1e-30
+    c = wcomp.compress(_on_gpu(codec.f32_to_bf16_rne(w)), CH=32)
+    plain = rng.standard_normal((T, K)).astype(np.float32)
+    spread = plain.copy()
+    spread[:, rng.permutation(K)[:K // 2]] *= np.float32(2.0 ** -40)
+    rows = np.zeros(T, bool)
+    rows[[3, 70, 71, 130, T - 1]] = True
+    mixed = np.where(rows[:, None], spread, plain)
+    y0 = torch.from_numpy(rng.standard_normal((T, N)).astype(np.float32)).cuda()
+    out = []
+    for x in (plain, spread, mixed):
+        y = y0.clone()
+        prefill.matrix(torch.from_numpy(x).cuda(), c, y, add=bool(mode))
+        out.append(y)
+    r = torch.from_numpy(rows).cuda()
+    assert torch.equal(out[2][~r], out[0][~r]) and torch.equal(out[2][r], out[1][r])
+
+
 def test_sums_over_chunks_keep_their_accuracy():
     """K = 4096 unsplit: the norm of the error stays below 4e-7 of the output's
     (2.3e-7 measured; 5.9e-7 without the float32 sums over chunks of steps, 5e-5
