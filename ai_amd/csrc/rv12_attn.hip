@@ -701,15 +701,16 @@ __global__ __launch_bounds__(512) void k_prefill_attn(AttnParams p) {
         }
         mb = fmaxf(mb, __shfl_xor(mb, 16));
         mb = fmaxf(mb, __shfl_xor(mb, 32));
-        // finite from the first block with a position the token sees (block 0
-        // for every token of an unsplit range); before it nothing accumulates
+        // finite from the first block with a finite score of a position the token
+        // sees; before it every score is -inf, and adds nothing, or NaN (which
+        // fmaxf passes over), and stays
         const float mn = fmaxf(m, mb);
-        const bool none = mn == -INFINITY;
-        const float alpha = none ? 1.0f : expf(m - mn);
+        const float mr = mn == -INFINITY ? 0.0f : mn;
+        const float alpha = expf(m - mr);
         float ls = 0.0f;
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-            pr[r] = none ? 0.0f : expf(sc[r] - mn);
+            pr[r] = expf(sc[r] - mr);
             ls += pr[r];
         }
         l = l * alpha + ls;
@@ -770,8 +771,9 @@ __global__ __launch_bounds__(512) void k_prefill_attn(AttnParams p) {
         for (int w = 1; w < PW; ++w) {
             const float* d = lds + ((w - 1) * G + hd) * kPart;
             const float mw = d[DT * 256 + lane], lw = d[DT * 256 + 64 + lane];
-            const float mn = fmaxf(m, mw);  // (part 0 has position 0, which every token sees)
-            const float a0 = expf(m - mn), a1 = mw == -INFINITY ? 0.0f : expf(mw - mn);
+            const float mn = fmaxf(m, mw);
+            // (a part without a finite score: its sums are zero, or NaN and stay so)
+            const float a0 = m == -INFINITY ? 0.0f : expf(m - mn), a1 = mw == -INFINITY ? 0.0f : expf(mw - mn);
 #pragma unroll
             for (int i = 0; i < DT; ++i) o[i] = o[i] * a0 + *reinterpret_cast<const f32x4*>(d + i * 256 + lane * 4) * a1;
             l = l * a0 + lw * a1;

@@ -632,3 +632,44 @@ def test_prefill_attention_with_more_waves_than_blocks(H, KV, HD, T, p0):
         vmax = float(vc[:, :p0 + T].float().abs().max())
         tol = (HD + p0 + T) * 2.0 ** -23 * HD ** 0.5 * vmax  # |score| <= sqrt(HD) |k| bound folded into one factor
         assert float((out - ref).abs().max()) <= tol, (dt, float((out - ref).abs().max()), tol)
+
+
+@pytest.mark.parametrize("H,KV,HD", [(8, 8, 64), (16, 8, 128), (32, 8, 128)])
+@pytest.mark.parametrize("what", ["nan_block_1", "nan_own", "inf_blocks"])
+@pytest.mark.parametrize("T,p0", [(16, 40), (40, 0), (70, 60)])
+def test_prefill_attention_keeps_nan_and_infinite_scores(H, KV, HD, what, T, p0):
+    """Keys that make whole blocks of scores NaN, a token's own key NaN (the only
+    position of its block that the first token of a block sees), and keys with an
+    infinity (scores of -inf for half the tokens over the first two blocks): NaN where
+    the float64 softmax has it, the others as in the tests above; the batched pass
+    alike.  At the shortest blocks most waves of a head have one such block alone.
+    (Infinite keys in a float32 cache only: with a bf16 cache q goes in parts of
+    either sign, and their products with an infinity cancel to NaN.)"""
+    from ai_amd.attn import RopeAttn
+    dev = "cuda"
+    g = torch.Generator(device=dev).manual_seed(T + HD)
+    for dt in (torch.float32,) if what == "inf_blocks" else (torch.float32, torch.bfloat16):
+        print("case", H, KV, HD, what, T, p0, dt, flush=True)
+        maxt = p0 + T + 5
+        qkv = torch.randn(T, (H + 2 * KV) * HD, device=dev, generator=g)
+        one, inv = torch.ones(HD, device=dev), torch.zeros(HD // 2, device=dev)  # no rotation: q is its RMSNorm
+        kc = torch.randn(KV, maxt, HD, device=dev, generator=g).to(dt)
+        vc = torch.randn(KV, maxt, HD, device=dev, generator=g).to(dt)
+        if what == "nan_own":
+            qkv.view(T, H + 2 * KV, HD)[T - T % 16 if T % 16 else 0, H:H + KV] = float("nan")
+        elif p0:
+            if what == "nan_block_1":
+                kc[:, 16:32] = float("nan")
+            else:
+                kc[:, :32, 3] = float("inf")
+        out, pos = torch.empty(T, H * HD, device=dev), torch.tensor([p0], device=dev)
+        a = RopeAttn(H, KV, HD, maxt, dt, 1e-6, dev)
+        kb, vb = kc.clone(), vc.clone()
+        a.prefill(qkv, one, one, inv, pos, kc, vc, out, T)
+        q = qkv.view(T, H + 2 * KV, HD)[:, :H].double()
+        q = q / torch.sqrt((q * q).mean(-1, keepdim=True) + 1e-6)
+        ref = _prefill_ref(q, kc, vc, p0, T, H, KV, HD)
+        assert torch.allclose(out, ref, rtol=1e-4, atol=1e-5, equal_nan=True)
+        if T <= 16:
+            a.batch(qkv, one, one, inv, pos, kb, vb, out, T)
+            assert torch.allclose(out, ref, rtol=1e-4, atol=1e-5, equal_nan=True)
