@@ -327,7 +327,7 @@ __global__ __launch_bounds__(kPfThreads) void k_prefill_mm(const uint32_t* __res
                                                            const float* __restrict__ ev, const float* __restrict__ xt,
                                                            int tp, const float* __restrict__ R, float* __restrict__ y,
                                                            float* __restrict__ part, int N, int K, int T, int add,
-                                                           int parts) {
+                                                           int parts, int vec) {
     extern __shared__ u32x4 bs[];  // the ring's slots: A tiles and B parts of consecutive steps
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -586,9 +586,9 @@ __global__ __launch_bounds__(kPfThreads) void k_prefill_mm(const uint32_t* __res
     // rs with RMS, stored or added; with a K split the split's sums go to
     // part[sp][token][row] instead (rs and the store or add are the reduce
     // pass's).  Loads that depend on nothing are issued together ahead of their
-    // use, and four rows of a token are one 16-byte load or store where
-    // N % 4 == 0 (indexes clamped into the matrix instead of branches; what is
-    // read past an edge is not stored): with a load, branch and store per value
+    // use, and four rows of a token are one 16-byte load or store where vec says
+    // that all of them are aligned (indexes clamped into the matrix instead of
+    // branches; what is read past an edge is not stored): with a load, branch and store per value
     // the pass took about 20 us of a workgroup, longer than 8 K steps.
     const int q = lane >> 4, jj = lane & 15;
     const int64_t rlo = blk0 * 16;
@@ -596,8 +596,7 @@ __global__ __launch_bounds__(kPfThreads) void k_prefill_mm(const uint32_t* __res
     asm volatile("" ::: "memory");
     if (rlo >= N || (wide ? ww : ~ww) == 0) return;  // nothing of this pass to store
     const int32_t e_lo = rp[rlo], e_hi = rp[min(rlo + 16 * kPfWB, (int64_t)N)];
-    const bool vec = (N & 3) == 0;  // y, part and rbase are 16-byte aligned
-    int64_t nr[kPfWB];              // the lane's first row of each tile
+    int64_t nr[kPfWB];  // the lane's first row of each tile
     int sc[kPfWB][4];
 #pragma unroll
     for (int b = 0; b < kPfWB; ++b) {
@@ -819,8 +818,11 @@ void launch_prefill(const rv12_matrix& w, const float* x, float* y, int T, int m
     const auto kern = lnw ? k_prefill_mm<true> : k_prefill_mm<false>;
     (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
                               (int)kPfLds);
+    // four rows at a time: rows of y and part start 16-byte aligned (their bases are,
+    // the caller's rbase may not be)
+    const int vec = N % 4 == 0 && reinterpret_cast<uintptr_t>(w.rbase) % 16 == 0;
     hipLaunchKernelGGL(kern, grid, dim3(kPfThreads), kPfLds, st, reinterpret_cast<const uint32_t*>(w.tiles), w.rbase, xb,
-                       E, w.rp, w.er, w.ec, w.ev, xt, tp, R, y, part, N, K, T, mode != 0 ? 1 : 0, parts);
+                       E, w.rp, w.er, w.ec, w.ev, xt, tp, R, y, part, N, K, T, mode != 0 ? 1 : 0, parts, vec);
     if (S > 1) {
         const int V = N % 4 == 0 ? 4 : 1;
         const dim3 rgrid((unsigned)((N + 256 * V - 1) / (256 * V)), (unsigned)min(T, 65535));

@@ -332,6 +332,25 @@ def test_a_token_does_not_depend_on_its_neighbours(N, K, T, mode):
     assert torch.equal(out[2][~r], out[0][~r]) and torch.equal(out[2][r], out[1][r])
 
 
+@pytest.mark.parametrize("N", [256, 300])
+def test_row_windows_at_any_four_byte_address(N):
+    """rbase has the alignment of its type: the same outputs from a copy that starts
+    4, 8 and 12 bytes past a 16-byte boundary."""
+    from ai_amd import prefill, wcomp
+    rng = np.random.default_rng(N)
+    w = (rng.standard_normal((N, 256)) * 0.02 * 2.0 ** rng.integers(-9, 9, (N, 1))).astype(np.float32)
+    c = wcomp.compress(_on_gpu(codec.f32_to_bf16_rne(w)))
+    x = torch.from_numpy(rng.standard_normal((33, 256)).astype(np.float32)).cuda()
+    y = torch.zeros(4, 33, N, device="cuda")
+    rb = c["q16_rbase"]
+    for off in range(4):
+        room = torch.empty(N + 4, dtype=torch.int32, device="cuda")
+        c["q16_rbase"] = room[off:off + N].copy_(rb)
+        assert c["q16_rbase"].data_ptr() % 16 == 4 * off
+        prefill.matrix(x, c, y[off], add=True)
+    assert torch.equal(y[1:], y[:1].expand(3, -1, -1)) and bool(y[0].any())
+
+
 def test_sums_over_chunks_keep_their_accuracy():
     """K = 4096 unsplit: the norm of the error stays below 4e-7 of the output's
     (2.3e-7 measured; 5.9e-7 without the float32 sums over chunks of steps, 5e-5
