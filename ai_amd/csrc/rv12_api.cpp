@@ -444,13 +444,13 @@ int rv12_encode_exc(const uint16_t* w, int n, int k, int base, const int32_t* rp
     return launch_status();
 }
 
-size_t rv12_compress_workspace_bytes(int n, int k) { return shape_ok(n, k) ? compress_ws_bytes(n) : 0; }
+size_t rv12_compress_workspace_bytes(int n, int k) { return shape_ok(n, k) ? compress_ws_bytes(n, k) : 0; }
 
 int rv12_compress_plan(const uint16_t* w, int n, int k, int32_t* rbase, int32_t* rp, int32_t* qrp, int32_t* out,
                        void* ws, size_t ws_bytes, void* stream) {
     if (!w || !rbase || !rp || !qrp || !out) return RV12_E_NULL;
     if (!shape_ok(n, k)) return RV12_E_SHAPE;
-    if (!ws || ws_bytes < compress_ws_bytes(n)) return RV12_E_WORKSPACE;
+    if (!ws || ws_bytes < compress_ws_bytes(n, k)) return RV12_E_WORKSPACE;
     if (!aligned16(w) || !aligned16(ws)) return RV12_E_ALIGN;
     launch_compress_plan(w, n, k, rbase, rp, qrp, out, ws, (hipStream_t)stream);
     return launch_status();

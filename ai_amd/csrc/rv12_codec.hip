@@ -7,10 +7,11 @@
 //            that layout's own exception list (k_row_windows, k_pack_tiles,
 //            k_exceptions)
 //   compress the packed form and the reference codec's base, row pointers and
-//            exception list together (k_row_windows, k_hist_sum, k_row_counts,
-//            k_row_pointers, k_pack_tiles, k_exceptions with both lists): two
-//            reads of the weights, a third of the rows with entries, one host
-//            read between (6144 x 4096: 79 us, 377 as separate calls)
+//            exception list together (k_row_windows, k_hist_sum, k_row_counts /
+//            k_row_recount, k_row_pointers, k_pack_tiles, k_exceptions with both
+//            lists): two reads of the weights (three of short rows), one more of
+//            the rows with entries, one host read between (6144 x 4096: 79 us,
+//            377 as separate calls)
 //   decode   Q16 rows back to the exact bf16 / float32 values (k_decode,
 //            k_decode_exc)
 // The Q16 layout and the h encoding are described in rv12_device.h.
@@ -330,11 +331,8 @@ __global__ __launch_bounds__(256) void k_hist_sum(const int32_t* __restrict__ pa
     if (t < kHistBins) hist[bin] = red[t];
 }
 
-// The matrix's own window (every workgroup finds it, by the same rule) and each
-// row's weights outside it, from the row's prefix counts.
-__global__ __launch_bounds__(256) void k_row_counts(const int64_t* __restrict__ hist, const int32_t* __restrict__ cs,
-                                                    int N, int K, int32_t* __restrict__ row_exc,
-                                                    int32_t* __restrict__ out) {
+// The matrix's own window from its histogram, by the rows' rule (a workgroup of 256)
+__device__ __forceinline__ int matrix_base(const int64_t* __restrict__ hist) {
     __shared__ int64_t h[256];
     __shared__ int64_t red[4];
     const int t = threadIdx.x;
@@ -350,13 +348,45 @@ __global__ __launch_bounds__(256) void k_row_counts(const int64_t* __restrict__ 
     for (int o = 32; o >= 1; o >>= 1) key = max(key, (int64_t)__shfl_xor((long long)key, o));
     if ((t & 63) == 0) red[t >> 6] = key;
     __syncthreads();
-    const int base = 255 - (int)(max(max(red[0], red[1]), max(red[2], red[3])) & 255);
-    const int n = blockIdx.x * 256 + t;
+    return 255 - (int)(max(max(red[0], red[1]), max(red[2], red[3])) & 255);
+}
+
+// The matrix's window (every workgroup finds it) and each row's weights outside
+// it, from the row's prefix counts.
+__global__ __launch_bounds__(256) void k_row_counts(const int64_t* __restrict__ hist, const int32_t* __restrict__ cs,
+                                                    int N, int K, int32_t* __restrict__ row_exc,
+                                                    int32_t* __restrict__ out) {
+    const int base = matrix_base(hist);
+    const int n = blockIdx.x * 256 + threadIdx.x;
     if (n < N) {
         const int32_t* r = cs + (int64_t)n * 256;
         row_exc[n] = K - (r[base + 14] - (base > 0 ? r[base - 1] : 0));
     }
     if (n == 0) out[0] = base;
+}
+
+// The same from the weights, 16 lanes per row, for rows that are shorter than their
+// prefix counts would be useful (kCountColumns).
+__global__ __launch_bounds__(256) void k_row_recount(const int64_t* __restrict__ hist, const uint16_t* __restrict__ w,
+                                                     int N, int K, int32_t* __restrict__ row_exc,
+                                                     int32_t* __restrict__ out) {
+    const int base = matrix_base(hist);
+    const int l = threadIdx.x & 15;
+    for (int n = blockIdx.x * 16 + (threadIdx.x >> 4); n < N; n += gridDim.x * 16) {
+        const uint16_t* row = w + (int64_t)n * K;
+        int cnt = 0;
+        for (int k = l * 8; k < K; k += 128) {
+            const uint4 v = *reinterpret_cast<const uint4*>(row + k);
+            const uint32_t d[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                cnt += ((d[j] >> 7 & 0xFF) - (uint32_t)base > 14u) + ((d[j] >> 23 & 0xFF) - (uint32_t)base > 14u);
+        }
+#pragma unroll
+        for (int o = 8; o >= 1; o >>= 1) cnt += __shfl_xor(cnt, o);
+        if (l == 0) row_exc[n] = cnt;
+    }
+    if (blockIdx.x == 0 && threadIdx.x == 0) out[0] = base;
 }
 
 // One workgroup: the row pointers of both exception lists from the rows' counts
@@ -507,12 +537,12 @@ void launch_codec_to_bf16(const rv12_codec& c, uint16_t* w, hipStream_t st) {
                            c.ev, c.n_exc, c.n, c.k, w);
 }
 
+static int row_grid(int N) { return min((N + kRowWaves - 1) / kRowWaves, kRowGrid); }
 static void launch_row_windows(const uint16_t* w, int N, int K, int32_t* rbase, int32_t* row_exc, int32_t* cs,
                                int32_t* part, hipStream_t st) {
     (void)hipFuncSetAttribute(reinterpret_cast<const void*>(k_row_windows), hipFuncAttributeMaxDynamicSharedMemorySize,
                               (int)kRowLds);
-    hipLaunchKernelGGL(k_row_windows, dim3((unsigned)min((N + kRowWaves - 1) / kRowWaves, kRowGrid)),
-                       dim3(kRowWaves * 64), kRowLds, st, w, N, K, rbase, row_exc, cs, part);
+    hipLaunchKernelGGL(k_row_windows, dim3((unsigned)row_grid(N)), dim3(kRowWaves * 64), kRowLds, st, w, N, K, rbase, row_exc, cs, part);
 }
 
 void launch_pack_plan(const uint16_t* w, int N, int K, int32_t* rbase, int32_t* row_exc, hipStream_t st) {
@@ -531,21 +561,32 @@ void launch_pack(const uint16_t* w, int N, int K, const int32_t* rbase, const in
     if (n_exc > 0) launch_exceptions(w, N, K, ExcList{rbase, 0, rp, er, ec, ev}, nullptr, st);
 }
 
-// the histogram and its parts, each row's entries in both lists, row prefix counts
+// Workspace: the histogram and its parts, each row's entries in both lists, and
+// from kCountColumns columns on the row prefix counts, 1 KB a row: no more there than
+// the 1.5 bytes per weight of m8 / e4 that the separate calls hold beside the tiles.
+// Shorter rows are counted again instead (65536 x 672: 69 MB at most beside the
+// weights and 194 us, 136 MB and 184 us with prefix counts; 135 MB as separate calls).
+constexpr int kCountColumns = 688;
 static size_t padded4(int N) { return ((size_t)N + 3) / 4 * 4; }
-size_t compress_ws_bytes(int N) { return 256 * 8 + ((size_t)kRowGrid * 256 + 2 * padded4(N) + (size_t)N * 256) * 4; }
+size_t compress_ws_bytes(int N, int K) {
+    return 256 * 8 + ((size_t)row_grid(N) * 256 + 2 * padded4(N) + (K >= kCountColumns ? (size_t)N * 256 : 0)) * 4;
+}
 
 void launch_compress_plan(const uint16_t* w, int N, int K, int32_t* rbase, int32_t* rp, int32_t* qrp, int32_t* out,
                           void* ws, hipStream_t st) {
     int64_t* hist = static_cast<int64_t*>(ws);
     int32_t* part = reinterpret_cast<int32_t*>(hist + 256);
-    int32_t* exc = part + (size_t)kRowGrid * 256;
+    int32_t* exc = part + (size_t)row_grid(N) * 256;
     int32_t* qexc = exc + padded4(N);
-    int32_t* cs = qexc + padded4(N);
+    int32_t* cs = K >= kCountColumns ? qexc + padded4(N) : nullptr;
     launch_row_windows(w, N, K, rbase, qexc, cs, part, st);
     hipLaunchKernelGGL(k_hist_sum, dim3(256 / kHistBins), dim3(256), 0, st, part,
-                       min((N + kRowWaves - 1) / kRowWaves, kRowGrid), hist);
-    hipLaunchKernelGGL(k_row_counts, dim3((unsigned)((N + 255) / 256)), dim3(256), 0, st, hist, cs, N, K, exc, out);
+                       row_grid(N), hist);
+    if (cs)
+        hipLaunchKernelGGL(k_row_counts, dim3((unsigned)((N + 255) / 256)), dim3(256), 0, st, hist, cs, N, K, exc, out);
+    else
+        hipLaunchKernelGGL(k_row_recount, dim3((unsigned)min((N + 15) / 16, 2048)), dim3(256), 0, st, hist, w, N, K, exc,
+                           out);
     hipLaunchKernelGGL(k_row_pointers, dim3(1), dim3(kPlanThreads), 0, st, exc, qexc, N, rp, qrp, out);
 }
 

@@ -202,7 +202,7 @@ void launch_pack(const uint16_t* w, int N, int K, const int32_t* rbase, const in
                  int32_t* er, int32_t* ec, float* ev, int64_t n_exc, hipStream_t st);
 void launch_decode(const rv12_matrix& w, int first, int last, void* out, int out_f32, hipStream_t st, int64_t e0,
                    int64_t e1);
-size_t compress_ws_bytes(int N);
+size_t compress_ws_bytes(int N, int K);
 void launch_compress_plan(const uint16_t* w, int N, int K, int32_t* rbase, int32_t* rp, int32_t* qrp, int32_t* out,
                           void* ws, hipStream_t st);
 void launch_compress_write(const uint16_t* w, int N, int K, int base, const int32_t* rp, int32_t* er, int32_t* ec,

@@ -417,3 +417,14 @@ def test_attention_wrapper_checks_the_caches():
             a.batch(qkv, qn, kn, inv, pos, good, good, out, 2)
         with pytest.raises(ValueError, match="int64"):
             a(qkv, qn, kn, inv, pos.int(), good, good, out)
+
+
+@pytest.mark.parametrize("k", [32, 256, 512, 672, 704, 4096])
+@pytest.mark.parametrize("n", [1, 300, 65536, 300000])
+def test_compress_workspace_is_below_the_arrays_of_the_separate_calls(n, k):
+    """At most 1.5 bytes per weight (the m8 and e4 that the separate calls hold)
+    plus 8 bytes a row, its two counts, and the histogram's parts, 1 KB per workgroup
+    of four rows, at most 512."""
+    from ai_amd import _lib
+    got = _lib.lib().rv12_compress_workspace_bytes(n, k)
+    assert 0 < got <= n * k * 3 // 2 + 8 * (n + 3) + 1024 * min((n + 3) // 4, 512) + 2048

@@ -180,7 +180,8 @@ def test_random_draws_against_the_oracle_codec():
         assert np.array_equal(back, bits), d
 
 
-@pytest.mark.parametrize("N,K,every", [(1, 32, 1), (3, 2080, 7), (17, 512, 0), (2050, 96, 5), (4097, 64, 1), (9000, 32, 40)])
+@pytest.mark.parametrize("N,K,every", [(1, 32, 1), (3, 2080, 7), (17, 512, 0), (2050, 96, 5), (4097, 64, 1), (9000, 32, 40),
+                                       (70, 672, 9), (70, 704, 9)])
 def test_compress_in_one_pass_matches_the_separate_calls(N, K, every):
     """base, row pointers, both exception lists, windows and tiles of compress()
     equal those of rv12_encode* and rv12_pack* called one after the other and
