@@ -5,6 +5,7 @@ cache untouched, and measured results are cached per library + device and
 read back into CFG1 / CFGT in the reference's (BN, w, S) format."""
 import json
 
+import numpy as np
 import pytest
 
 from ai_amd import tune, wcomp
@@ -89,3 +90,18 @@ def test_rms_shapes_measured_with_the_prologue_and_cached_apart(fake, tmp_path):
     tune.tune([(6144, 4096, 0)], log=lambda *a: None, cache=str(p))  # the plain shape is measured on its own
     assert len(seen) > n
     assert set(json.loads(p.read_text())["entries"]) == {"6144x4096|0|rms", "4096x12288|2", "6144x4096|0"}
+
+
+def test_launches_are_looked_up_by_value():
+    """A launch triple held in mutable scalars, changed between calls, resolves to
+    the values it has at each call; equal numbers of any type share one entry."""
+    import torch
+    from ai_amd import wcomp
+    w, s = torch.tensor(4), np.array(1)
+    assert wcomp._resolved(1024, 2048, 1, 32, w, s)[0].waves == 4
+    w.fill_(8)
+    s[...] = 2
+    cfg = wcomp._resolved(1024, 2048, 1, np.int64(32), w, s)[0]
+    assert (cfg.waves, cfg.splits) == (8, 2)
+    n = len(wcomp._RESOLVED)
+    assert wcomp._resolved(1024, 2048, 1, 32.0, np.int32(8), 2)[0] is cfg and len(wcomp._RESOLVED) == n
