@@ -26,6 +26,7 @@ Launch parameters keep the reference meaning: BN = rows per workgroup
 (rounded up to 16, 32 or 64), w = waves per workgroup, S = K splits.
 """
 import ctypes
+import operator
 
 import torch
 
@@ -119,6 +120,7 @@ def compress(W, CH=256):
     if W.dtype != torch.bfloat16 or W.dim() != 2:
         raise ValueError("W must be a 2-D bfloat16 tensor")
     N, K = W.shape
+    CH = operator.index(CH)
     assert K % CH == 0
     dev = W.device
     W = W.contiguous()
@@ -159,7 +161,8 @@ def _compress_packed(W, N, K, CH, dev):
 
 def _compress_arrays(W, N, K, CH, dev):
     """compress() of a matrix without a packed form (K or CH off its steps), whose
-    dict keeps m8 and e4."""
+    dict keeps m8 and e4; or, by the separate calls, of one that has it (from 2^20
+    columns on, where pack() says that there are too many)."""
     st = _stream(dev)
     L = lib()
     hist = torch.empty(256, dtype=torch.int32, device=dev)
@@ -178,7 +181,7 @@ def _compress_arrays(W, N, K, CH, dev):
     if E:
         check(L.rv12_encode_exc(_ptr(W), N, K, base, _ptr(rp), _ptr(er), _ptr(ec), _ptr(ev), st), "compress")
     c = Codec12(base=base, rp=rp, er=er, ec=ec, ev=ev, N=N, K=K, CH=CH)
-    if CH > 0 and K % 32 == 0 and CH % 16 == 0:
+    if K % 32 == 0 and CH % 16 == 0:
         c.update(pack(W))
     else:  # no packed form for this K: the dict keeps the reference arrays
         c["m8"], c["e4"] = m8, e4

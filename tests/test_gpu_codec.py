@@ -208,3 +208,13 @@ def test_compress_in_one_pass_matches_the_separate_calls(N, K, every):
     for k in ("rp", "er", "ec"):
         assert np.array_equal(c[k].cpu().numpy(), o[k]), k
     assert np.array_equal(c["ev"].cpu().numpy().view(np.uint32), np.asarray(o["ev"]).view(np.uint32))
+
+
+def test_chunk_sizes_are_whole_numbers():
+    """A float chunk size is refused, whichever way the matrix would take."""
+    from ai_amd import wcomp
+    W = torch.ones(4, 96, dtype=torch.bfloat16, device="cuda")
+    for CH in (32.0, 24.0):
+        with pytest.raises(TypeError):
+            wcomp.compress(W, CH=CH)
+    assert type(wcomp.compress(W, CH=np.int64(32))["CH"]) is int
