@@ -19,8 +19,9 @@ reads each weight once in its 12-bit packed form (the Q16 tiles are the
 MFMA's A operand), accumulates in fp32 and adds the
 exceptions; no wider copy of W is ever written.  The reference computes the
 same sums with IEEE fp32 products after decoding W to fp32
-(prefill_kernels.py:8-26, 58-110); both are fp32 evaluations of the same
-closed form, held to the same error bound in the tests.
+(prefill_kernels.py:8-26, 58-110); the tests hold both to the error bound of an
+fp32 evaluation of the closed form, each output against the sum of its products'
+magnitudes.  A token's outputs depend on its own row and on the number of tokens.
 
 The q/k head norms, RoPE, the cache writes and the attention over the prompt
 (qk_rope_cache_k, tkernels.py:82-150, and att_k, prefill_kernels.py:29-54)
@@ -73,18 +74,19 @@ def _linear(x, c, y, mode, lnw=None, eps=1e-6, parts=2):
         _WS[key] = torch.empty(need, dtype=torch.uint8, device=x.device)
     ws = _WS[key]
     rc = L.rv12_prefill_linear_parts(ctypes.byref(wcomp._matrix(c)), ctypes.c_void_p(x.data_ptr()),
-                               ctypes.c_void_p(y.data_ptr()), T,
-                               None if lnw is None else ctypes.c_void_p(lnw.data_ptr()), float(eps), int(mode), parts,
-                               ctypes.c_void_p(ws.data_ptr()), ws.numel(),
-                               ctypes.c_void_p(torch.cuda.current_stream(x.device).cuda_stream))
+                                     ctypes.c_void_p(y.data_ptr()), T,
+                                     None if lnw is None else ctypes.c_void_p(lnw.data_ptr()), float(eps), int(mode),
+                                     parts, ctypes.c_void_p(ws.data_ptr()), ws.numel(),
+                                     ctypes.c_void_p(torch.cuda.current_stream(x.device).cuda_stream))
     _lib.check(rc, "prefill")
 
 
-def matrix(x, c, y, add=False, lnw=None, eps=1e-6):
+def matrix(x, c, y, add=False, lnw=None, eps=1e-6, parts=2):
     """y (=|+=) x . W^T for every token row of x (fp32 [T, K]); W read once
     in its 12-bit form (prefill.py:66-78).  lnw: the rows' RMSNorm (rmsg_k,
-    prefill.py:94) fused into the linear."""
-    _linear(x, c, y, 1 if add else 0, lnw, eps)
+    prefill.py:94) fused into the linear.  parts: 2 16-bit parts per activation
+    (23 bits, sums over chunks: the smaller error) or 3 (all 24 bits of each)."""
+    _linear(x, c, y, 1 if add else 0, lnw, eps, parts)
 
 
 _ATT = {}  # (dimensions, cache, device) -> RopeAttn launch parameters and workspace
@@ -123,8 +125,9 @@ def layer(eng, l, weights, x, start, kc, vc, gguf=False):
     s = eng.small[l]
     bf = lambda t: t.to(torch.bfloat16).contiguous()
     qkv = torch.empty(T, (H + 2 * KV) * HD, device=x.device)
-    # three parts: the keys and values rounded into the cache stay bit for bit
-    # what earlier prompts left there
+    # three parts: a layer's keys and values, rounded into its cache, are bit for
+    # bit what earlier versions left there for the same x (in a whole prompt: layer
+    # 0, as x itself differs in its last bits from then on)
     _linear(x, W["qkv"], qkv, 0, bf(s["ln1"]), eps, parts=3)
     f32 = lambda t: t.float().contiguous()
     att = torch.empty(T, H * HD, device=x.device)

@@ -380,7 +380,8 @@ def _resolved(N, K, T, BN, w, S):
     that depend on these six numbers alone (taken as plain integers: a tensor scalar
     would be looked up by its identity, an array not at all).  An invalid one
     raises each time."""
-    BN, w, S = None if BN is None else int(BN), int(w or 0), int(S or 0)
+    if not (BN is w is S is None):
+        BN, w, S = None if BN is None else int(BN), int(w or 0), int(S or 0)
     key = (N, K, T, BN, w, S)
     r = _RESOLVED.get(key)
     if r is None:

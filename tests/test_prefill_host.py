@@ -22,8 +22,8 @@ def test_enabled_follows_the_reference_variables(monkeypatch):
 
 
 def test_prefill_workspace_bytes():
-    """Ten bytes per column and token (three bf16 parts and the transposed
-    fp32 x'), tokens padded to 128, plus a scale exponent and an RMS factor per
+    """Ten bytes per column and token (room for three 16-bit parts, and the
+    transposed fp32 x'), tokens padded to 128, plus a scale exponent and an RMS factor per
     padded token; with a K split, a float per split, padded token and row for
     the partial sums: none for the Qwen3-8B gu and o over 2048 tokens (six
     rounds of workgroups, one full round), between 2 and 16 splits for the o
