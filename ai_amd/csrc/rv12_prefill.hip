@@ -27,22 +27,26 @@
 //      2.5e-7 against 2.4e-7, 7.0e-7, 1.5e-6).  A token whose values the float16
 //      parts would not hold (see tok_exp) keeps the three bf16 parts, whatever the
 //      others of its tile do, and so do all tokens of a call that asks for them
-//      (parts = 3): the prompt's qkv, whose keys and values are rounded into the
-//      cache and must stay, bit for bit, what earlier prompts left there (with two
-//      parts one in 10^4 bf16 entries falls on the other side of its rounding; the
-//      three parts cost the Qwen3-8B layer over 2048 tokens about 40 us of 2036).
+//      (parts = 3): the prompt's qkv, so that a layer leaves the same keys and
+//      values in its cache, bit for bit, as earlier versions did for the same x
+//      (layer 0 of a prompt; with two parts one in 10^4 bf16 entries falls on the
+//      other side of its rounding, 5e-5 of the layer's keys and values).  That is
+//      not for accuracy: one accumulator over K has the larger error, and the
+//      Qwen3-8B layer over 2048 tokens takes about 40 us more.
 //      Workgroup = 256 rows x 128 tokens, 8 waves of 64 rows x 64 tokens.  Per
 //      32-column step the workgroup's 16 row blocks' Q16 tiles and the B parts
 //      go from memory straight into a ring of LDS slots (buffer loads with the
 //      LDS destination), one wait + barrier per step; every other instruction
 //      is spread between the MFMAs.
-//      Bound by the matrix cores at the clock that the power limit leaves:
-//      51200 x 5120 over 4096 tokens is 2.15e12 useful operations and twice
-//      that in MFMAs, 5560 us with three parts and 4000 with two: the matrix
-//      cores are busy about half of the cycles at 1.8 GHz, and a library's
-//      bf16 product of that shape reaches 1.17 PFLOP/s where this does 1.07.
-//      (256-token workgroups, whose waves read a sixth less from LDS per
-//      product, took 3590 us, but leave no registers for the second sums:
+//      Bound by issue: 51200 x 5120 over 4096 tokens, 2.15e12 useful operations
+//      and twice that in MFMAs, takes 4100-4200 us (5560 with three parts), 1.05
+//      PFLOP/s of MFMAs.  Of a step's 1960 cycles the two waves of a SIMD have it
+//      issue MFMAs in 1024 and other vector instructions (the unpacking, the
+//      scaling, addresses: 100 a wave) in 800; LDS is active in 27 %, without bank
+//      conflicts; the clock under this load is 1.78 GHz (counters of this
+//      kernel).  A library's product of that shape reaches 1.17 PFLOP/s in bf16,
+//      1.13 in float16.  (256-token workgroups, whose waves unpack and read less
+//      per product, were 11 % faster, but leave no registers for the second sums:
 //      their error stays at 5.9e-7.)
 #include <hip/hip_runtime.h>
 #include <limits.h>
@@ -88,8 +92,8 @@ constexpr int kPfWait2 = kPfOps2 * (kPfRing2 - 3);
 // matrix core's own additions into an accumulator lose more as it grows: all
 // 128 steps of K = 4096 in one accumulator leave a relative error of 5.9e-7
 // against 64 bits (7.0e-7 with three bf16 parts), chunks of 16 steps 2.3e-7,
-// of 8 1.9e-7, of 4 1.7e-7; 51200 x 5120 over 4096 tokens takes 4310, 4115,
-// 4170 and 4290 us.
+// of 8 1.9e-7, of 4 1.7e-7; 51200 x 5120 over 4096 tokens took 4310, 4115,
+// 4170 and 4290 us (before the second part was scaled; 2 % more since).
 constexpr int kPfChunk = 16;
 // bf16 loop: 3 parts, four 40 KB slots
 constexpr int kPfRing3 = 4;
