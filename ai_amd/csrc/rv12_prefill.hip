@@ -12,9 +12,10 @@
 //   1. k_prefill_stats (one wave per token): the exponents of x' and, with
 //      RMS, rs (sum of squares of x 2^-32); k_prefill_parts (32 tokens x 64
 //      columns per workgroup): x' 2^P_t split into parts in B-operand lane
-//      order (token block, step of 32 columns, part, 64 lanes x 8 values; lane
-//      l: token l%16, k = 8(l/16) + 0..7), and x' itself in fp32, transposed
-//      (column-major over the padded tokens).  Token rows past T are zeros.
+//      order (token block; the first two parts of each step of 32 columns, then
+//      the third ones; 64 lanes x 8 values, lane l: token l%16, k = 8(l/16) +
+//      0..7), and x' itself in fp32, transposed (column-major over the padded
+//      tokens).  Token rows past T are zeros.
 //   2. k_prefill_mm: a 12-bit weight is exactly a float16 (4 exponent bits, 7
 //      of mantissa), so x' goes in two float16 parts (23 bits) with two MFMAs per
 //      tile where three bf16 parts (24 bits) took three.  The second part is kept
@@ -39,7 +40,7 @@
 //      LDS destination), one wait + barrier per step; every other instruction
 //      is spread between the MFMAs.
 //      Bound by issue: 51200 x 5120 over 4096 tokens, 2.15e12 useful operations
-//      and twice that in MFMAs, takes 4100-4200 us (5560 with three parts), 1.05
+//      and twice that in MFMAs, takes 4030 us (5560 with three parts), 1.07
 //      PFLOP/s of MFMAs.  Of a step's 1960 cycles the two waves of a SIMD have it
 //      issue MFMAs in 1024 and other vector instructions (the unpacking, the
 //      scaling, addresses: 100 a wave) in 800; LDS is active in 27 %, without bank
@@ -92,8 +93,8 @@ constexpr int kPfWait2 = kPfOps2 * (kPfRing2 - 3);
 // matrix core's own additions into an accumulator lose more as it grows: all
 // 128 steps of K = 4096 in one accumulator leave a relative error of 5.9e-7
 // against 64 bits (7.0e-7 with three bf16 parts), chunks of 16 steps 2.3e-7,
-// of 8 1.9e-7, of 4 1.7e-7; 51200 x 5120 over 4096 tokens took 4310, 4115,
-// 4170 and 4290 us (before the second part was scaled; 2 % more since).
+// of 8 1.9e-7, of 4 1.7e-7; in one sweep 51200 x 5120 over 4096 tokens took 4310,
+// 4115, 4170 and 4290 us.
 constexpr int kPfChunk = 16;
 // bf16 loop: 3 parts, four 40 KB slots
 constexpr int kPfRing3 = 4;
