@@ -281,7 +281,8 @@ def _on_gpu(bits):
     return torch.from_numpy(bits.view(np.int16)).view(torch.bfloat16).cuda()
 
 
-@pytest.mark.parametrize("K,low", [(32, 17), (64, 34), (480, 14), (544, 300), (4096, 200), (4096, 2200)])
+@pytest.mark.parametrize("K,low", [(32, 17), (64, 34), (480, 14), (544, 1), (544, 300), (4096, 8),
+                                   (4096, 113), (4096, 200), (4096, 2200)])
 @pytest.mark.parametrize("drop", [14, 20, 25, 28, 36, 60])
 def test_tokens_of_two_levels(K, low, drop):
     """`low` columns 2^drop below the others, in every third token, and rows with
