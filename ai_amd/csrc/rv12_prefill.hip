@@ -167,11 +167,12 @@ __device__ __forceinline__ int scale_bf16(int E) {
     return (e >= -39 && e <= kXRangeHi) ? kXScaleExp : slow_scale_exp(e);
 }
 
-// which of the tokens t0 .. t0 + 63 are wide (t0 < T; past T: as the last one)
-__device__ __forceinline__ uint64_t wide_mask(int E) { return __ballot(E & 1); }
+// E of the lane's token of t0 .. t0 + 63 (past T: the last one), and which of the
+// wave's 64 are wide
 __device__ __forceinline__ int class_of(const int* __restrict__ E, int t0, int T) {
     return E[min(t0 + (int)(threadIdx.x & 63), T - 1)];
 }
+__device__ __forceinline__ uint64_t wide_mask(int E) { return __ballot(E & 1); }
 
 // 1a. k_prefill_stats: one wave per token (4 per workgroup, a grid over the
 // padded tokens): the largest and smallest exponent of the nonzero x' and, with
@@ -407,322 +408,322 @@ __global__ __launch_bounds__(kPfThreads) void k_prefill_mm(const uint32_t* __res
     const uint64_t w0 = parts == 3 ? ~0ull : wide_mask(wl0), w1 = parts == 3 ? ~0ull : wide_mask(wl1);
     const uint64_t ww = wc ? w1 : w0;  // the wave's 64 tokens
     auto tile_pass = [&](auto wide_c) {
-    constexpr bool wide = decltype(wide_c)::value;
-    f32x4 acc[kPfWB][kPfWT];
-#pragma unroll
-    for (int b = 0; b < kPfWB; ++b)
-#pragma unroll
-        for (int c = 0; c < kPfWT; ++c) acc[b][c] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-
-    if constexpr (!wide) {
-        const int ra0 = wr * kPfWB * 64 + lane, rb0 = kPfSlotA + wc * kPfWT * 128 + lane;
-        auto read_a = [&](int slot, int b) { return *reinterpret_cast<const u32x3*>(bs + slot + ra0 + b * 64); };
-        // fragment i: part i / kPfWT of token block i % kPfWT, so that the products
-        // of one accumulator are kPfWT fragments apart
-        auto read_b = [&](int slot, int i) { return bs[slot + rb0 + (i % kPfWT) * 128 + (i / kPfWT) * 64]; };
-        // steps 0 and 1 landed
-        asm volatile("" ::: "memory");
-        __builtin_amdgcn_s_waitcnt(waitcnt_vm(kPfWait2));
-        __builtin_amdgcn_s_barrier();
-        asm volatile("" ::: "memory");
-        u32x4 a[2][kPfWB], up[kPfWB], fb[W];  // up: the step's weights times 2^11, for the hi parts
-#pragma unroll
-        for (int b = 0; b < kPfWB; ++b) {
-            const u32x3 r = read_a(0, b);
-            uint32_t pr[4];
-            unpack_pairs_f16(r.x, r.y, r.z, pr);
-            a[0][b] = u32x4{pr[0], pr[1], pr[2], pr[3]};
-        }
-#pragma unroll
-        for (int i = 0; i < W; ++i) fb[i] = read_b(0, i);
-        // Step s: wait for this wave's loads of step s + 1; barrier (every
-        // wave's have landed, and every wave has used slot s - 1); then per B
-        // fragment its four MFMAs, one of the loads of step s + kPfRing2 - 1 into
-        // slot s - 1, the read of the fragment W ahead (the next step's at the
-        // end) and a share of the next step's A reads and unpacking: memory,
-        // LDS and vector instructions spread between the MFMAs, fenced so
-        // that the compiler keeps them there.
-        int cur = 0, nxt = kPfSlot2, fill = (kPfRing2 - 1) * kPfSlot2;
-        const int nst = s_hi - s_lo;
-        f32x4 sum[kPfWB][kPfWT];
+        constexpr bool wide = decltype(wide_c)::value;
+        f32x4 acc[kPfWB][kPfWT];
 #pragma unroll
         for (int b = 0; b < kPfWB; ++b)
 #pragma unroll
-            for (int c = 0; c < kPfWT; ++c) sum[b][c] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-        for (int s1 = 0; s1 < nst; s1 += kPfChunk) {
-            const int s2 = min(nst, s1 + kPfChunk);
-            for (int s0 = s1; s0 < s2; s0 += 2) {
+            for (int c = 0; c < kPfWT; ++c) acc[b][c] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+
+        if constexpr (!wide) {
+            const int ra0 = wr * kPfWB * 64 + lane, rb0 = kPfSlotA + wc * kPfWT * 128 + lane;
+            auto read_a = [&](int slot, int b) { return *reinterpret_cast<const u32x3*>(bs + slot + ra0 + b * 64); };
+            // fragment i: part i / kPfWT of token block i % kPfWT, so that the products
+            // of one accumulator are kPfWT fragments apart
+            auto read_b = [&](int slot, int i) { return bs[slot + rb0 + (i % kPfWT) * 128 + (i / kPfWT) * 64]; };
+            // steps 0 and 1 landed
+            asm volatile("" ::: "memory");
+            __builtin_amdgcn_s_waitcnt(waitcnt_vm(kPfWait2));
+            __builtin_amdgcn_s_barrier();
+            asm volatile("" ::: "memory");
+            u32x4 a[2][kPfWB], up[kPfWB], fb[W];  // up: the step's weights times 2^11, for the hi parts
 #pragma unroll
-                for (int u = 0; u < 2; ++u) {
-                    asm volatile("" ::: "memory");
-                    __builtin_amdgcn_s_waitcnt(waitcnt_vm(kPfWait2));
-                    __builtin_amdgcn_s_barrier();
-                    asm volatile("" ::: "memory");
-                    u32x3 raw[kPfWB];
+            for (int b = 0; b < kPfWB; ++b) {
+                const u32x3 r = read_a(0, b);
+                uint32_t pr[4];
+                unpack_pairs_f16(r.x, r.y, r.z, pr);
+                a[0][b] = u32x4{pr[0], pr[1], pr[2], pr[3]};
+            }
 #pragma unroll
-                    for (int i = 0; i < kFrags; ++i) {
-                        if (i < kPfOps2) load_op(i, fill, s0 + u + kPfRing2 - 1);
-                        if (i >= 1 && i - 1 < kPfWB) raw[i - 1] = read_a(nxt, i - 1);
-                        const u32x4 bf = fb[i % W];
+            for (int i = 0; i < W; ++i) fb[i] = read_b(0, i);
+            // Step s: wait for this wave's loads of step s + 1; barrier (every
+            // wave's have landed, and every wave has used slot s - 1); then per B
+            // fragment its four MFMAs, one of the loads of step s + kPfRing2 - 1 into
+            // slot s - 1, the read of the fragment W ahead (the next step's at the
+            // end) and a share of the next step's A reads and unpacking: memory,
+            // LDS and vector instructions spread between the MFMAs, fenced so
+            // that the compiler keeps them there.
+            int cur = 0, nxt = kPfSlot2, fill = (kPfRing2 - 1) * kPfSlot2;
+            const int nst = s_hi - s_lo;
+            f32x4 sum[kPfWB][kPfWT];
 #pragma unroll
-                        for (int b = 0; b < kPfWB; ++b)
-                            acc[b][i % kPfWT] = mfma_f16(i < kPfWT ? a[u][b] : up[b], bf, acc[b][i % kPfWT]);
-                        if (i < kPfWB) up[i] = f16_up11(a[u][i]);
-                        fb[i % W] = i + W < kFrags ? read_b(cur, i + W) : read_b(nxt, i + W - kFrags);
-                        if (i >= kFrags - kPfWB) {
-                            const int b = i - (kFrags - kPfWB);
-                            uint32_t pr[4];
-                            unpack_pairs_f16(raw[b].x, raw[b].y, raw[b].z, pr);
-                            a[u ^ 1][b] = u32x4{pr[0], pr[1], pr[2], pr[3]};
+            for (int b = 0; b < kPfWB; ++b)
+#pragma unroll
+                for (int c = 0; c < kPfWT; ++c) sum[b][c] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+            for (int s1 = 0; s1 < nst; s1 += kPfChunk) {
+                const int s2 = min(nst, s1 + kPfChunk);
+                for (int s0 = s1; s0 < s2; s0 += 2) {
+#pragma unroll
+                    for (int u = 0; u < 2; ++u) {
+                        asm volatile("" ::: "memory");
+                        __builtin_amdgcn_s_waitcnt(waitcnt_vm(kPfWait2));
+                        __builtin_amdgcn_s_barrier();
+                        asm volatile("" ::: "memory");
+                        u32x3 raw[kPfWB];
+#pragma unroll
+                        for (int i = 0; i < kFrags; ++i) {
+                            if (i < kPfOps2) load_op(i, fill, s0 + u + kPfRing2 - 1);
+                            if (i >= 1 && i - 1 < kPfWB) raw[i - 1] = read_a(nxt, i - 1);
+                            const u32x4 bf = fb[i % W];
+#pragma unroll
+                            for (int b = 0; b < kPfWB; ++b)
+                                acc[b][i % kPfWT] = mfma_f16(i < kPfWT ? a[u][b] : up[b], bf, acc[b][i % kPfWT]);
+                            if (i < kPfWB) up[i] = f16_up11(a[u][i]);
+                            fb[i % W] = i + W < kFrags ? read_b(cur, i + W) : read_b(nxt, i + W - kFrags);
+                            if (i >= kFrags - kPfWB) {
+                                const int b = i - (kFrags - kPfWB);
+                                uint32_t pr[4];
+                                unpack_pairs_f16(raw[b].x, raw[b].y, raw[b].z, pr);
+                                a[u ^ 1][b] = u32x4{pr[0], pr[1], pr[2], pr[3]};
+                            }
+                            __builtin_amdgcn_sched_barrier(0);
                         }
-                        __builtin_amdgcn_sched_barrier(0);
+                        fill = cur;
+                        cur = nxt;
+                        nxt = nxt + kPfSlot2 == kPfRing2 * kPfSlot2 ? 0 : nxt + kPfSlot2;
                     }
-                    fill = cur;
-                    cur = nxt;
-                    nxt = nxt + kPfSlot2 == kPfRing2 * kPfSlot2 ? 0 : nxt + kPfSlot2;
                 }
+#pragma unroll
+                for (int b = 0; b < kPfWB; ++b)
+#pragma unroll
+                    for (int c = 0; c < kPfWT; ++c) {
+                        sum[b][c] += acc[b][c];
+                        acc[b][c] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+                    }
             }
 #pragma unroll
             for (int b = 0; b < kPfWB; ++b)
 #pragma unroll
-                for (int c = 0; c < kPfWT; ++c) {
-                    sum[b][c] += acc[b][c];
-                    acc[b][c] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+                for (int c = 0; c < kPfWT; ++c) acc[b][c] = sum[b][c];
+        } else {
+            // the first loads have landed, and a first pass's LDS accesses are done
+            asm volatile("" ::: "memory");
+            __builtin_amdgcn_s_waitcnt(waitcnt_vm_lgkm0(0));
+            __builtin_amdgcn_s_barrier();
+            asm volatile("" ::: "memory");
+            int boff3[3], bstep3[3];
+#pragma unroll
+            for (int j = 0; j < 3; ++j) {
+                const int ch = wave + j * kPfWaves, pt = ch % 3;  // (token block, part) of the step
+                boff3[j] = ((ch / 3 * 192 + (pt < 2 ? 0 : 128)) * nsteps + (pt & 1) * 64 + lane) * 16;
+                bstep3[j] = pt < 2 ? 128 * 16 : 64 * 16;
+            }
+            int need = 0;  // the wave's token blocks with a wide token
+#pragma unroll
+            for (int c = 0; c < kPfWT; ++c) need |= (ww >> (16 * c) & 0xFFFF) != 0 ? 1 << c : 0;
+            auto load_step = [&](int slot, int j) {  // step s_lo + j
+                const int s = s_lo + j;
+                const bool in = s < s_hi;
+                const __amdgpu_buffer_rsrc_t ra = in ? rv : rnull, rb = in ? rbx : rbnull;
+                const int sa = (in ? s : 0) * kStepBytes, sb = in ? s : 0;
+                u32x4* d = bs + slot * kPfSlot3;
+#pragma unroll
+                for (int i = 0; i < kPfAPerWave; ++i)
+                    load_lds12(ra, d + (wave * kPfAPerWave + i) * 64, aoff[i], sa);
+#pragma unroll
+                for (int j = 0; j < 3; ++j)
+                    load_lds16(rb, d + kPfSlotA + wave * 64 + j * kPfThreads, boff3[j], sb * bstep3[j]);
+            };
+            // this wave's fragments of the step in slot `slot`: its 4 row blocks' A
+            // groups and 3 parts x 4 token blocks of B, part-major so the first
+            // part's MFMAs wait only for its own reads
+            auto read_frags = [&](u32x3 (&fa)[kPfWB], u32x4 (&fb)[3][kPfWT], int slot) {
+                const u32x4* d = bs + slot * kPfSlot3;
+#pragma unroll
+                for (int b = 0; b < kPfWB; ++b) fa[b] = *reinterpret_cast<const u32x3*>(d + (wr * kPfWB + b) * 64 + lane);
+                const u32x4* src = d + kPfSlotA + wc * kPfWT * 192 + lane;
+#pragma unroll
+                for (int c = 0; c < kPfWT; ++c)
+                    if (need >> c & 1)
+#pragma unroll
+                        for (int q = 0; q < 3; ++q) fb[q][c] = src[c * 192 + q * 64];
+            };
+            // steps 0-3 into slots 0-3, all landed; step 0's fragments read
+#pragma unroll
+            for (int i = 0; i < kPfRing3; ++i) load_step(i, i);
+            asm volatile("" ::: "memory");
+            __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));
+            __builtin_amdgcn_s_barrier();
+            asm volatile("" ::: "memory");
+            u32x3 fa[2][kPfWB];
+            u32x4 fb[2][3][kPfWT];
+            read_frags(fa[0], fb[0], 0);
+            // Step s: wait for this wave's loads of step s + 1 and its fragment reads
+            // of step s; barrier; step s + 4 into slot s % 4; the fragments of step
+            // s + 1 read while the 48 MFMAs of step s run (12 for each token block that
+            // has a wide token).  Whole rounds of the unroll: steps past the split read
+            // zeros and add nothing.
+            for (int s0 = 0; s0 < s_hi - s_lo; s0 += kPfRing3) {
+#pragma unroll
+                for (int u = 0; u < kPfRing3; ++u) {
+                    asm volatile("" ::: "memory");
+                    __builtin_amdgcn_s_waitcnt(waitcnt_vm_lgkm0(kPfWait3));
+                    __builtin_amdgcn_s_barrier();
+                    asm volatile("" ::: "memory");
+                    load_step(u, s0 + u + kPfRing3);
+                    read_frags(fa[(u + 1) & 1], fb[(u + 1) & 1], (u + 1) % kPfRing3);
+                    asm volatile("" ::: "memory");
+                    __builtin_amdgcn_sched_barrier(0);
+                    u32x4 a[kPfWB];
+#pragma unroll
+                    for (int b = 0; b < kPfWB; ++b) {
+                        uint32_t pr[4];
+                        unpack_pairs(fa[u & 1][b].x, fa[u & 1][b].y, fa[u & 1][b].z, pr);
+                        a[b] = u32x4{pr[0], pr[1], pr[2], pr[3]};
+                    }
+#pragma unroll
+                    for (int c = 0; c < kPfWT; ++c) {
+                        if (!(need >> c & 1)) continue;
+#pragma unroll
+                        for (int q = 0; q < 3; ++q)
+#pragma unroll
+                            for (int b = 0; b < kPfWB; ++b) acc[b][c] = mfma(a[b], fb[u & 1][q][c], acc[b][c]);
+                    }
                 }
+            }
         }
-#pragma unroll
-        for (int b = 0; b < kPfWB; ++b)
-#pragma unroll
-            for (int c = 0; c < kPfWT; ++c) acc[b][c] = sum[b][c];
-    } else {
-        // the first loads have landed, and a first pass's LDS accesses are done
-        asm volatile("" ::: "memory");
-        __builtin_amdgcn_s_waitcnt(waitcnt_vm_lgkm0(0));
-        __builtin_amdgcn_s_barrier();
-        asm volatile("" ::: "memory");
-        int boff3[3], bstep3[3];
-#pragma unroll
-        for (int j = 0; j < 3; ++j) {
-            const int ch = wave + j * kPfWaves, pt = ch % 3;  // (token block, part) of the step
-            boff3[j] = ((ch / 3 * 192 + (pt < 2 ? 0 : 128)) * nsteps + (pt & 1) * 64 + lane) * 16;
-            bstep3[j] = pt < 2 ? 128 * 16 : 64 * 16;
-        }
-        int need = 0;  // the wave's token blocks with a wide token
-#pragma unroll
-        for (int c = 0; c < kPfWT; ++c) need |= (ww >> (16 * c) & 0xFFFF) != 0 ? 1 << c : 0;
-        auto load_step = [&](int slot, int j) {  // step s_lo + j
-            const int s = s_lo + j;
-            const bool in = s < s_hi;
-            const __amdgpu_buffer_rsrc_t ra = in ? rv : rnull, rb = in ? rbx : rbnull;
-            const int sa = (in ? s : 0) * kStepBytes, sb = in ? s : 0;
-            u32x4* d = bs + slot * kPfSlot3;
-#pragma unroll
-            for (int i = 0; i < kPfAPerWave; ++i)
-                load_lds12(ra, d + (wave * kPfAPerWave + i) * 64, aoff[i], sa);
-#pragma unroll
-            for (int j = 0; j < 3; ++j)
-                load_lds16(rb, d + kPfSlotA + wave * 64 + j * kPfThreads, boff3[j], sb * bstep3[j]);
-        };
-        // this wave's fragments of the step in slot `slot`: its 4 row blocks' A
-        // groups and 3 parts x 4 token blocks of B, part-major so the first
-        // part's MFMAs wait only for its own reads
-        auto read_frags = [&](u32x3 (&fa)[kPfWB], u32x4 (&fb)[3][kPfWT], int slot) {
-            const u32x4* d = bs + slot * kPfSlot3;
-#pragma unroll
-            for (int b = 0; b < kPfWB; ++b) fa[b] = *reinterpret_cast<const u32x3*>(d + (wr * kPfWB + b) * 64 + lane);
-            const u32x4* src = d + kPfSlotA + wc * kPfWT * 192 + lane;
-#pragma unroll
-            for (int c = 0; c < kPfWT; ++c)
-                if (need >> c & 1)
-#pragma unroll
-                    for (int q = 0; q < 3; ++q) fb[q][c] = src[c * 192 + q * 64];
-        };
-        // steps 0-3 into slots 0-3, all landed; step 0's fragments read
-#pragma unroll
-        for (int i = 0; i < kPfRing3; ++i) load_step(i, i);
+        // the last loads (zeros into slots nobody reads) land before the
+        // workgroup's LDS can be handed on
         asm volatile("" ::: "memory");
         __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));
-        __builtin_amdgcn_s_barrier();
-        asm volatile("" ::: "memory");
-        u32x3 fa[2][kPfWB];
-        u32x4 fb[2][3][kPfWT];
-        read_frags(fa[0], fb[0], 0);
-        // Step s: wait for this wave's loads of step s + 1 and its fragment reads
-        // of step s; barrier; step s + 4 into slot s % 4; the fragments of step
-        // s + 1 read while the 48 MFMAs of step s run (12 for each token block that
-        // has a wide token).  Whole rounds of the unroll: steps past the split read
-        // zeros and add nothing.
-        for (int s0 = 0; s0 < s_hi - s_lo; s0 += kPfRing3) {
-#pragma unroll
-            for (int u = 0; u < kPfRing3; ++u) {
-                asm volatile("" ::: "memory");
-                __builtin_amdgcn_s_waitcnt(waitcnt_vm_lgkm0(kPfWait3));
-                __builtin_amdgcn_s_barrier();
-                asm volatile("" ::: "memory");
-                load_step(u, s0 + u + kPfRing3);
-                read_frags(fa[(u + 1) & 1], fb[(u + 1) & 1], (u + 1) % kPfRing3);
-                asm volatile("" ::: "memory");
-                __builtin_amdgcn_sched_barrier(0);
-                u32x4 a[kPfWB];
-#pragma unroll
-                for (int b = 0; b < kPfWB; ++b) {
-                    uint32_t pr[4];
-                    unpack_pairs(fa[u & 1][b].x, fa[u & 1][b].y, fa[u & 1][b].z, pr);
-                    a[b] = u32x4{pr[0], pr[1], pr[2], pr[3]};
-                }
-#pragma unroll
-                for (int c = 0; c < kPfWT; ++c) {
-                    if (!(need >> c & 1)) continue;
-#pragma unroll
-                    for (int q = 0; q < 3; ++q)
-#pragma unroll
-                        for (int b = 0; b < kPfWB; ++b) acc[b][c] = mfma(a[b], fb[u & 1][q][c], acc[b][c]);
-                }
-            }
-        }
-    }
-    // the last loads (zeros into slots nobody reads) land before the
-    // workgroup's LDS can be handed on
-    asm volatile("" ::: "memory");
-    __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));
 
-    // epilogue: lane l holds token 16 c + l%16 and rows 4(l/16) + 0..3 of each
-    // tile.  v = acc 2^(sc_row - P_t) (exact), plus the row's exceptions, times
-    // rs with RMS, stored or added; with a K split the split's sums go to
-    // part[sp][token][row] instead (rs and the store or add are the reduce
-    // pass's).  Loads that depend on nothing are issued together ahead of their
-    // use, and four rows of a token are one 16-byte load or store where vec says
-    // that all of them are aligned (indexes clamped into the matrix instead of
-    // branches; what is read past an edge is not stored): with a load, branch and store per value
-    // the pass took about 20 us of a workgroup, longer than 8 K steps.
-    const int q = lane >> 4, jj = lane & 15;
-    const int64_t rlo = blk0 * 16;
-    __builtin_amdgcn_s_barrier();  // the ring's LDS is the exception sums' from here
-    asm volatile("" ::: "memory");
-    if (rlo >= N || (wide ? ww : ~ww) == 0) return;  // nothing of this pass to store
-    const int32_t e_lo = rp[rlo], e_hi = rp[min(rlo + 16 * kPfWB, (int64_t)N)];
-    int64_t nr[kPfWB];  // the lane's first row of each tile
-    int sc[kPfWB][4];
-#pragma unroll
-    for (int b = 0; b < kPfWB; ++b) {
-        nr[b] = rlo + b * 16 + q * 4;
-        if (vec) {
-            const int4 r = *reinterpret_cast<const int4*>(rbase + min(nr[b], (int64_t)N - 4));
-            sc[b][0] = r.x, sc[b][1] = r.y, sc[b][2] = r.z, sc[b][3] = r.w;
-        } else {
-#pragma unroll
-            for (int i = 0; i < 4; ++i) sc[b][i] = rbase[min(nr[b] + i, (int64_t)N - 1)];
-        }
-    }
-    float* xs = reinterpret_cast<float*>(bs) + wave * (16 * kPfWB * kPfExcStride);  // the wave's [64 rows][64 tokens]
-    const int tbw = tb0 + wc * kPfWT;  // the wave's token blocks
-    // (a) v = acc 2^(sc_row - P_t), exact
-#pragma unroll
-    for (int c = 0; c < kPfWT; ++c) {
-        const int et = E[min((tbw + c) * 16 + jj, T - 1)];
-        const int pt = wide ? scale_bf16(et) : scale_f16(et) + kF16WeightExp + 11;
-#pragma unroll
-        for (int b = 0; b < kPfWB; ++b)
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-                acc[b][c][i] = ldexpf(acc[b][c][i], scale_exp(sc[b][i]) - pt);
-    }
-    // (b) the exceptions of the wave's 64 rows (the tiles hold zeros
-    // there) added in list order, lane = token: the sums go through LDS, an
-    // entry's row, column and value are wave-uniform (scalar loads), x' of
-    // the 64 tokens at its column is 256 contiguous bytes of the transposed
-    // copy, and a row's sums stay in a register from its first entry to its
-    // last.  (With a K split, the entries whose column lies in the split's
-    // steps.)  One wave's LDS accesses stay in order; the fences keep the
-    // compiler's in theirs.
-    if (e_lo < e_hi) {
-        constexpr int EB = 8;
-#pragma unroll
-        for (int b = 0; b < kPfWB; ++b)
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int c = 0; c < kPfWT; ++c)
-                    xs[(b * 16 + q * 4 + i) * kPfExcStride + c * 16 + jj] = acc[b][c][i];
+        // epilogue: lane l holds token 16 c + l%16 and rows 4(l/16) + 0..3 of each
+        // tile.  v = acc 2^(sc_row - P_t) (exact), plus the row's exceptions, times
+        // rs with RMS, stored or added; with a K split the split's sums go to
+        // part[sp][token][row] instead (rs and the store or add are the reduce
+        // pass's).  Loads that depend on nothing are issued together ahead of their
+        // use, and four rows of a token are one 16-byte load or store where vec says
+        // that all of them are aligned (indexes clamped into the matrix instead of
+        // branches; what is read past an edge is not stored): with a load, branch and store per value
+        // the pass took about 20 us of a workgroup, longer than 8 K steps.
+        const int q = lane >> 4, jj = lane & 15;
+        const int64_t rlo = blk0 * 16;
+        __builtin_amdgcn_s_barrier();  // the ring's LDS is the exception sums' from here
         asm volatile("" ::: "memory");
-        const float* xtw = xt + (int64_t)tbw * 16 + lane;
-        const int c_lo = s_lo * 32, c_hi = s_hi * 32;
-        int row = 0;
-        float sum = xs[lane];
-        for (int32_t e0 = e_lo; e0 < e_hi; e0 += EB) {
-            int r[EB];
-            float g[EB], v[EB];
-#pragma unroll
-            for (int j = 0; j < EB; ++j) {
-                const int32_t e = min(e0 + j, e_hi - 1);
-                const int col = ec[e];
-                const bool in = e0 + j < e_hi && col >= c_lo && col < c_hi;
-                r[j] = in ? (int)(er[e] - rlo) : -1;
-                v[j] = ev[e];
-                g[j] = xtw[(int64_t)col * tp];
-            }
-#pragma unroll
-            for (int j = 0; j < EB; ++j) {
-                if (r[j] < 0) continue;
-                if (r[j] != row) {
-                    xs[row * kPfExcStride + lane] = sum;
-                    row = r[j];
-                    sum = xs[row * kPfExcStride + lane];
-                }
-                sum += v[j] * g[j];
-            }
-        }
-        xs[row * kPfExcStride + lane] = sum;
-        asm volatile("" ::: "memory");
-#pragma unroll
-        for (int b = 0; b < kPfWB; ++b)
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int c = 0; c < kPfWT; ++c)
-                    acc[b][c][i] = xs[(b * 16 + q * 4 + i) * kPfExcStride + c * 16 + jj];
-    }
-    // (c) the outputs
-    int tok[kPfWT];
-    float rs[kPfWT];
-    f32x4 oy[kPfWB][kPfWT];
-#pragma unroll
-    for (int c = 0; c < kPfWT; ++c) {
-        tok[c] = (tbw + c) * 16 + jj;
-        const int tc = min(tok[c], T - 1);
-        rs[c] = LN && S == 1 ? R[tc] : 1.0f;
-        const float* yr = y + (int64_t)tc * N;
+        if (rlo >= N || (wide ? ww : ~ww) == 0) return;  // nothing of this pass to store
+        const int32_t e_lo = rp[rlo], e_hi = rp[min(rlo + 16 * kPfWB, (int64_t)N)];
+        int64_t nr[kPfWB];  // the lane's first row of each tile
+        int sc[kPfWB][4];
 #pragma unroll
         for (int b = 0; b < kPfWB; ++b) {
-            oy[b][c] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-            if (add && S == 1) {
-                if (vec) {
-                    oy[b][c] = *reinterpret_cast<const f32x4*>(yr + min(nr[b], (int64_t)N - 4));
-                } else {
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) oy[b][c][i] = yr[min(nr[b] + i, (int64_t)N - 1)];
-                }
-            }
-        }
-    }
-#pragma unroll
-    for (int c = 0; c < kPfWT; ++c) {
-        float* dst = S > 1 ? part + ((int64_t)sp * tp + tok[c]) * N : y + (int64_t)tok[c] * N;
-#pragma unroll
-        for (int b = 0; b < kPfWB; ++b) {
-            f32x4 v = acc[b][c];
-            if constexpr (LN) v *= rs[c];
-            if (add && S == 1) v = oy[b][c] + v;
-            if (tok[c] >= T || (ww >> (16 * c + jj) & 1) != (wide ? 1 : 0)) continue;
+            nr[b] = rlo + b * 16 + q * 4;
             if (vec) {
-                if (nr[b] < N) *reinterpret_cast<f32x4*>(dst + nr[b]) = v;
+                const int4 r = *reinterpret_cast<const int4*>(rbase + min(nr[b], (int64_t)N - 4));
+                sc[b][0] = r.x, sc[b][1] = r.y, sc[b][2] = r.z, sc[b][3] = r.w;
             } else {
 #pragma unroll
-                for (int i = 0; i < 4; ++i)
-                    if (nr[b] + i < N) dst[nr[b] + i] = v[i];
+                for (int i = 0; i < 4; ++i) sc[b][i] = rbase[min(nr[b] + i, (int64_t)N - 1)];
             }
         }
-    }
+        float* xs = reinterpret_cast<float*>(bs) + wave * (16 * kPfWB * kPfExcStride);  // the wave's [64 rows][64 tokens]
+        const int tbw = tb0 + wc * kPfWT;  // the wave's token blocks
+        // (a) v = acc 2^(sc_row - P_t), exact
+#pragma unroll
+        for (int c = 0; c < kPfWT; ++c) {
+            const int et = E[min((tbw + c) * 16 + jj, T - 1)];
+            const int pt = wide ? scale_bf16(et) : scale_f16(et) + kF16WeightExp + 11;
+#pragma unroll
+            for (int b = 0; b < kPfWB; ++b)
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    acc[b][c][i] = ldexpf(acc[b][c][i], scale_exp(sc[b][i]) - pt);
+        }
+        // (b) the exceptions of the wave's 64 rows (the tiles hold zeros
+        // there) added in list order, lane = token: the sums go through LDS, an
+        // entry's row, column and value are wave-uniform (scalar loads), x' of
+        // the 64 tokens at its column is 256 contiguous bytes of the transposed
+        // copy, and a row's sums stay in a register from its first entry to its
+        // last.  (With a K split, the entries whose column lies in the split's
+        // steps.)  One wave's LDS accesses stay in order; the fences keep the
+        // compiler's in theirs.
+        if (e_lo < e_hi) {
+            constexpr int EB = 8;
+#pragma unroll
+            for (int b = 0; b < kPfWB; ++b)
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+#pragma unroll
+                    for (int c = 0; c < kPfWT; ++c)
+                        xs[(b * 16 + q * 4 + i) * kPfExcStride + c * 16 + jj] = acc[b][c][i];
+            asm volatile("" ::: "memory");
+            const float* xtw = xt + (int64_t)tbw * 16 + lane;
+            const int c_lo = s_lo * 32, c_hi = s_hi * 32;
+            int row = 0;
+            float sum = xs[lane];
+            for (int32_t e0 = e_lo; e0 < e_hi; e0 += EB) {
+                int r[EB];
+                float g[EB], v[EB];
+#pragma unroll
+                for (int j = 0; j < EB; ++j) {
+                    const int32_t e = min(e0 + j, e_hi - 1);
+                    const int col = ec[e];
+                    const bool in = e0 + j < e_hi && col >= c_lo && col < c_hi;
+                    r[j] = in ? (int)(er[e] - rlo) : -1;
+                    v[j] = ev[e];
+                    g[j] = xtw[(int64_t)col * tp];
+                }
+#pragma unroll
+                for (int j = 0; j < EB; ++j) {
+                    if (r[j] < 0) continue;
+                    if (r[j] != row) {
+                        xs[row * kPfExcStride + lane] = sum;
+                        row = r[j];
+                        sum = xs[row * kPfExcStride + lane];
+                    }
+                    sum += v[j] * g[j];
+                }
+            }
+            xs[row * kPfExcStride + lane] = sum;
+            asm volatile("" ::: "memory");
+#pragma unroll
+            for (int b = 0; b < kPfWB; ++b)
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+#pragma unroll
+                    for (int c = 0; c < kPfWT; ++c)
+                        acc[b][c][i] = xs[(b * 16 + q * 4 + i) * kPfExcStride + c * 16 + jj];
+        }
+        // (c) the outputs
+        int tok[kPfWT];
+        float rs[kPfWT];
+        f32x4 oy[kPfWB][kPfWT];
+#pragma unroll
+        for (int c = 0; c < kPfWT; ++c) {
+            tok[c] = (tbw + c) * 16 + jj;
+            const int tc = min(tok[c], T - 1);
+            rs[c] = LN && S == 1 ? R[tc] : 1.0f;
+            const float* yr = y + (int64_t)tc * N;
+#pragma unroll
+            for (int b = 0; b < kPfWB; ++b) {
+                oy[b][c] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+                if (add && S == 1) {
+                    if (vec) {
+                        oy[b][c] = *reinterpret_cast<const f32x4*>(yr + min(nr[b], (int64_t)N - 4));
+                    } else {
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) oy[b][c][i] = yr[min(nr[b] + i, (int64_t)N - 1)];
+                    }
+                }
+            }
+        }
+#pragma unroll
+        for (int c = 0; c < kPfWT; ++c) {
+            float* dst = S > 1 ? part + ((int64_t)sp * tp + tok[c]) * N : y + (int64_t)tok[c] * N;
+#pragma unroll
+            for (int b = 0; b < kPfWB; ++b) {
+                f32x4 v = acc[b][c];
+                if constexpr (LN) v *= rs[c];
+                if (add && S == 1) v = oy[b][c] + v;
+                if (tok[c] >= T || (ww >> (16 * c + jj) & 1) != (wide ? 1 : 0)) continue;
+                if (vec) {
+                    if (nr[b] < N) *reinterpret_cast<f32x4*>(dst + nr[b]) = v;
+                } else {
+#pragma unroll
+                    for (int i = 0; i < 4; ++i)
+                        if (nr[b] + i < N) dst[nr[b] + i] = v[i];
+                }
+            }
+        }
     };
     if ((w0 & w1) != ~0ull) tile_pass(std::false_type{});
     if ((w0 | w1) != 0) tile_pass(std::true_type{});
